@@ -19,8 +19,8 @@
 //    tile each) of one (batch, head): Q8 rows, S, P and the O^T accumulators
 //    (fp32, 32 x D) all live in arch VGPRs.
 //  * K8 rows and V^T rows reach LDS in tiles of 64 keys by direct global ->
-//    LDS loads (global_load_lds_dwordx4), three tiles ahead of their use, in a
-//    ring of 5 slots: no staging registers and no VALU work.  V arrives
+//    LDS loads (global_load_lds_dwordx4), two iterations ahead of their use, in
+//    a ring of K tiles and one of V tiles: no staging registers, no VALU work.  V arrives
 //    already converted and transposed (sage_vtiles), so a tile is a plain
 //    copy.  The 16-byte chunks of each LDS row are XOR-swizzled so that the
 //    operand reads of 16 consecutive lanes (rows) hit distinct banks.
@@ -254,14 +254,30 @@ __device__ __forceinline__ int swz(int r) {
 typedef __attribute__((address_space(1))) const void gmem_t;
 typedef __attribute__((address_space(3))) void lmem_t;
 
+// LDS rings of the tile loads.  Iteration j reads K tile j+1 and V tile j-1
+// while K tiles j+2, j+3 and V tiles j .. j+kVA arrive: at least 3 K slots and
+// 2 + kVA V slots, each tile requested at the start of the iteration before
+// the last one that may wait for it.  One ring of 5 K+V slots, three tiles
+// ahead for both, held every V tile two iterations longer than needed; the
+// two rings take 72 KB instead of 121 (INT8, D = 128, 16-bit V).  Whole calls,
+// alternating with the one ring: 925 -> 910 us at B4 H32 N4096 D128, 571 -> 563
+// at B8 H16 N4096 D64 (4-slot rings: a trip of the unrolled loop is 4
+// iterations, not 10), 1062 -> 1029 unquantized at B4 H32 N4096 D128.
+template <int QKM, int D, int PVM, int NW>
+struct TileRing {
+  static constexpr bool kI8 = QKM == kQkI8 || QKM == kQkI8Q;
+  static constexpr int NK = D == 64 ? 4 : 3;
+  static constexpr int NV = D == 64 ? 4 : (kI8 ? 3 : 2);
+  static constexpr int kVA = NV > 2 ? 1 : 0;
+};
+
 // One work-group: 8 waves (2 per SIMD) of 32 query rows (one 32-row MFMA tile
 // each) of one (batch, head); Q rows, S, P and the O^T accumulators live in
 // arch VGPRs.  Tiles of 64 keys (K rows and V^T rows) reach LDS by direct
-// global -> LDS loads, three tiles ahead of their use, in a ring of 5.
-template <int QKM, int D, int PVM, typename TO>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_kernel(AttnArgs a) {
-  constexpr int NW = 8;
-  constexpr int BM = 256;  // query rows per work-group
+// global -> LDS loads, two iterations ahead of their use (TileRing).
+template <int QKM, int D, int PVM, typename TO, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_kernel(AttnArgs a) {
+  constexpr int BM = 32 * NW;  // query rows per work-group
   constexpr bool kFQ = QKM == kQkI8Q;  // Q quantized in the prologue
   constexpr bool kI8 = QKM == kQkI8 || kFQ;
   constexpr bool kF8 = PVM == SAGE_PV_FP8;
@@ -276,21 +292,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int VRB = 64 * EB;      // V^T row bytes
   constexpr int KTB = kBN * KRB;    // K tile bytes
   constexpr int VTB = D * VRB;      // V^T tile bytes
-  constexpr int SLOT = KTB + VTB;
-  constexpr int NBUF = 5;           // tiles j-1 .. j+3 of iteration j
-  constexpr int KLD = KTB / 1024;   // 1 KB wave loads per K8 tile
+  using Ring = TileRing<QKM, D, PVM, NW>;
+  constexpr int NK = Ring::NK, NV = Ring::NV, kVA = Ring::kVA;
+  constexpr int VOFF = NK * KTB;                  // V tiles follow the K tiles
+  constexpr int RING = NK * KTB + NV * VTB;
+  constexpr int KLD = KTB / 1024;                 // 1 KB wave loads per K tile
   constexpr int VLD = VTB / 1024;
-  constexpr int LPW = (KLD + VLD + NW - 1) / NW;  // wave loads per wave per tile
-  static_assert(LPW * NW >= KLD + VLD && LPW <= 15, "tile loads");
-  constexpr int SINK = LPW * NW > KLD + VLD ? 1024 : 0;  // target of spare loads
+  constexpr int KPW = (KLD + NW - 1) / NW;        // of each wave
+  constexpr int VPW = (VLD + NW - 1) / NW;
+  constexpr int LPW = KPW + VPW;
+  static_assert(LPW <= 15, "tile loads");
+  constexpr int SINK = KPW * NW > KLD || VPW * NW > VLD ? 1024 : 0;  // target of spare loads
 
-  __shared__ __attribute__((aligned(1024))) char smem[NBUF * SLOT + SINK];
+  // One LDS array for everything: with a second __shared__ variable the
+  // compiler gives LDS accesses alias scopes, takes the operand reads of the
+  // ring for reads of the direct-to-LDS load issued last and drains the
+  // prefetch before them (an s_waitcnt vmcnt(0) per iteration).
+  constexpr int QAMAX = kFQ ? NW * (int)sizeof(float) : 0;  // the waves' max|x| of Q
+  __shared__ __attribute__((aligned(1024))) char smem[RING + SINK + QAMAX];
 #if SAGE_TRACE
   // stamps go to LDS as they are taken (kept in registers they would change
   // the kernel being measured; a global store would enter the vmcnt
   // accounting of the tile loads) and to the trace buffer at the end.  A
   // kernel whose tile ring leaves no room for them is not traced.
-  constexpr bool kTrace = NBUF * SLOT + SINK + NW * kTraceWords * 8 <= 160 * 1024;
+  constexpr bool kTrace = RING + SINK + QAMAX + NW * kTraceWords * 8 <= 160 * 1024;
   unsigned long long* tr_s = nullptr;
   if constexpr (kTrace) tr_s = trace_lds<NW>();
   // every lane stores the same wave-uniform value (no branch around the store)
@@ -389,84 +414,68 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (a.causal) nfull = min(nfull, (qa + 1) / kBN);
   nfull = min(nfull, jmax + 1);
 
-  // ---- tile loads.  Wave load g = wave + 8i (i < LPW) of a tile is the 1 KB
-  // LDS range [1024g, 1024g + 1024) of its slot (K8 rows first, then V^T rows);
-  // lane l brings the 16-byte chunk that lands at offset 16l, i.e. the logical
-  // chunk (physical chunk ^ swizzle of its row).  K8 rows past Nkv read the
-  // last row (their P is 0); V^T tiles are zero past Nkv.  Loads past the
-  // tile go to the sink, so every wave issues LPW loads per tile.
-  auto load_tile = [&](int j, int sl) __attribute__((always_inline)) {  // sl = j % NBUF
-    char* slot = smem + sl * SLOT;
-    const int k0 = j * kBN;
-    const uint8_t* vt = vtbase + (int64_t)j * VTB;
+  // ---- tile loads.  Wave load g = wave + NW*i of a K (V) tile is the 1 KB LDS
+  // range [1024g, 1024g + 1024) of its slot; lane l brings the 16-byte chunk
+  // that lands at offset 16l, i.e. the logical chunk (physical chunk ^ swizzle
+  // of its row).  K rows past Nkv read the last row (their P is 0); V tiles
+  // are zero past Nkv.  Loads past the tile go to the sink, so every
+  // wave issues KPW loads per K tile and VPW per V tile.  `whole`: every row
+  // of the tile is < Nkv, so each load is a uniform tile base plus a lane
+  // offset that does not change from tile to tile.
+  uint32_t kfoff[KPW], vfoff[VPW];
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) {
+  for (int i = 0; i < KPW; ++i) {
+    const int p = 64 * (wave + NW * i) + lane;
+    const int r = p / (KRB / 16), pc = p % (KRB / 16);
+    kfoff[i] = wave + NW * i < KLD ? (uint32_t)(r * a.skn * QEB + 16 * (pc ^ swz<KRB>(r))) : 0u;
+  }
+#pragma unroll
+  for (int i = 0; i < VPW; ++i) {
+    const int p = 64 * (wave + NW * i) + lane;
+    const int d = p / (VRB / 16), pc = p % (VRB / 16);
+    vfoff[i] = wave + NW * i < VLD ? (uint32_t)(d * VRB + 16 * (pc ^ swz<VRB>(d))) : 0u;
+  }
+  const int64_t ktile_bytes = (int64_t)kBN * a.skn * QEB;
+  auto load_k = [&](int j, int sl, bool whole) __attribute__((always_inline)) {  // sl = j % NK
+    char* slot = smem + sl * KTB;
+    const char* base = kbase + j * ktile_bytes;
+    asm("" : "+s"(base));  // an SGPR pair: the lane offsets stay 32-bit (no 64-bit lane addresses hoisted)
+#pragma unroll
+    for (int i = 0; i < KPW; ++i) {
       const int g = wave + NW * i;  // wave-uniform
-      const void* src;
-      char* dst;
-      if (g < KLD) {
+      const bool in = KLD % NW == 0 || g < KLD;
+      const char* src = in ? base + kfoff[i] : kbase;
+      if (!whole && in) {
         const int p = 64 * g + lane;
         const int r = p / (KRB / 16), pc = p % (KRB / 16);
-        const int row = min(k0 + r, a.Nkv - 1);
+        const int row = min(j * kBN + r, a.Nkv - 1);
         src = kbase + (uint32_t)(row * a.skn * QEB + 16 * (pc ^ swz<KRB>(r)));
-        dst = slot + 1024 * g;
-      } else if (g < KLD + VLD) {
-        const int p = 64 * (g - KLD) + lane;
-        const int d = p / (VRB / 16), pc = p % (VRB / 16);
-        src = vt + d * VRB + 16 * (pc ^ swz<VRB>(d));
-        dst = slot + KTB + 1024 * (g - KLD);
-      } else {  // only when SINK > 0
-        src = kbase;
-        dst = smem + NBUF * SLOT;
       }
+      char* dst = in ? slot + 1024 * g : smem + RING;
       __builtin_amdgcn_global_load_lds((gmem_t*)src, (lmem_t*)dst, 16, 0, 0);
     }
   };
-  // Tile loads of the mask-free loop: only whole K tiles (every row < Nkv),
-  // so each of the wave's LPW loads is a uniform tile base plus a lane offset
-  // that does not change from tile to tile.
-  uint32_t foff[LPW];
+  auto load_v = [&](int j, int sl) __attribute__((always_inline)) {  // sl = j % NV
+    char* slot = smem + VOFF + sl * VTB;
+    const char* base = reinterpret_cast<const char*>(vtbase) + (int64_t)j * VTB;
+    asm("" : "+s"(base));
 #pragma unroll
-  for (int i = 0; i < LPW; ++i) {
-    const int g = wave + NW * i;
-    if (g < KLD) {
-      const int p = 64 * g + lane;
-      const int r = p / (KRB / 16), pc = p % (KRB / 16);
-      foff[i] = (uint32_t)(r * a.skn * QEB + 16 * (pc ^ swz<KRB>(r)));
-    } else if (g < KLD + VLD) {
-      const int p = 64 * (g - KLD) + lane;
-      const int d = p / (VRB / 16), pc = p % (VRB / 16);
-      foff[i] = (uint32_t)(d * VRB + 16 * (pc ^ swz<VRB>(d)));
-    } else {
-      foff[i] = 0;
-    }
-  }
-  const int64_t ktile_bytes = (int64_t)kBN * a.skn * QEB;
-  auto load_tile_fast = [&](int j, int sl) __attribute__((always_inline)) {  // sl = j % NBUF
-    char* slot = smem + sl * SLOT;
-#pragma unroll
-    for (int i = 0; i < LPW; ++i) {
+    for (int i = 0; i < VPW; ++i) {
       const int g = wave + NW * i;  // wave-uniform
-      const char* base;
-      char* dst;
-      if (g < KLD) {
-        base = kbase + j * ktile_bytes;
-        dst = slot + 1024 * g;
-      } else if (g < KLD + VLD) {
-        base = reinterpret_cast<const char*>(vtbase) + (int64_t)j * VTB;
-        dst = slot + KTB + 1024 * (g - KLD);
-      } else {
-        base = kbase;
-        dst = smem + NBUF * SLOT;
-      }
-      __builtin_amdgcn_global_load_lds((gmem_t*)(base + foff[i]), (lmem_t*)dst, 16, 0, 0);
+      const bool in = VLD % NW == 0 || g < VLD;
+      const char* src = in ? base + vfoff[i] : kbase;
+      char* dst = in ? slot + 1024 * g : smem + RING;
+      __builtin_amdgcn_global_load_lds((gmem_t*)src, (lmem_t*)dst, 16, 0, 0);
     }
   };
-  // end of an iteration: this wave's loads of the tile needed next are done
-  // (at most `ahead` younger tiles in flight), its LDS reads are done, barrier
-  // (fast: called from the mask-free loops, for the trace's split)
-  auto sync_tiles = [&](bool ahead, bool fast = false) __attribute__((always_inline)) {
-    if (ahead) SAGE_WAIT_VM(LPW);
+  // end of iteration j: this wave's loads of K tile j+2 and V tile j are done
+  // (those issued in this iteration may be in flight: kahead K tile j+3,
+  // vahead V tile j + kVA), its LDS reads are done, barrier (fast: called
+  // from the mask-free loops, for the trace's split)
+  auto sync_tiles = [&](bool kahead, bool vahead, bool fast = false) __attribute__((always_inline)) {
+    if (kahead && vahead) SAGE_WAIT_VM(KPW + (kVA > 0 ? VPW : 0));
+    else if (kahead) SAGE_WAIT_VM(KPW);
+    else if (vahead && kVA > 0) SAGE_WAIT_VM(VPW);
     else SAGE_WAIT_VM(0);
 #if SAGE_TRACE >= 2
     const unsigned long long tb = __builtin_amdgcn_s_memtime();
@@ -532,13 +541,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int VCH = kF8 ? 2 : 4;  // chunks of a V^T operand read per d tile
   int voff[VCH];  // V^T row 32dt + n (swizzle independent of dt)
 #pragma unroll
-  for (int c = 0; c < VCH; ++c) voff[c] = KTB + n * VRB + 16 * ((VCH * hh + c) ^ swz<VRB>(n));
+  for (int c = 0; c < VCH; ++c) voff[c] = VOFF + n * VRB + 16 * ((VCH * hh + c) ^ swz<VRB>(n));
 
   // ---- building blocks
-  // S^T of block j (its K tile in slot j % NBUF): K row 32t + n, bytes 32c + 16hh
+  // S^T of block j (its K tile in slot j % NK): K row 32t + n, bytes 32c + 16hh
   // (into the S buffer Sd, its k scale into kd)
-  auto qk_into = [&](int j, int sl, SAcc (&Sd)[2], float& kd) __attribute__((always_inline)) {  // sl = j % NBUF
-    const char* ks = smem + sl * SLOT;
+  auto qk_into = [&](int j, int sl, SAcc (&Sd)[2], float& kd) __attribute__((always_inline)) {  // sl = j % NK
+    int so = sl * KTB;
+    if constexpr (D == 128) asm("" : "+s"(so));  // one SGPR, not an induction variable per operand offset
+    const char* ks = smem + so;
     if constexpr (kI8) kd = ksc_base[min(j >> a.blkk_shift, a.nks - 1)];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -561,9 +572,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   };
   auto qk = [&](int j, int sl) __attribute__((always_inline)) { qk_into(j, sl, S, ksc_cur); };
-  // O^T += V^T P^T of block j (its V^T tile in slot j % NBUF)
-  auto pv = [&](int sl, const uint32_t (&P)[PW]) __attribute__((always_inline)) {  // sl = j % NBUF
-    const char* vs = smem + sl * SLOT;
+  // O^T += V^T P^T of block j (its V tile in slot j % NV)
+  auto pv = [&](int sl, const uint32_t (&P)[PW]) __attribute__((always_inline)) {  // sl = j % NV
+    int so = sl * VTB;
+    if constexpr (D == 128) asm("" : "+s"(so));
+    const char* vs = smem + so;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       const char* vr = vs + 32 * dt * VRB;
@@ -773,39 +786,44 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // iterations.  The mask-free steady state has a loop of its own so that the
   // O accumulators are updated from one place in each loop.
   auto generic_iter = [&](int j) __attribute__((always_inline)) {
-    if (j + 3 < nkb) load_tile(j + 3, (j + 3) % NBUF);
+    if (j + kVA < nkb) load_v(j + kVA, (j + kVA) % NV);
+    if (j + 3 < nkb) load_k(j + 3, (j + 3) % NK, false);
     if (pend) {
       rescale_o();
       pend = false;
     }
-    if (j >= 1 && j - 1 <= jmax) pv((j - 1) % NBUF, Pprev);
+    if (j >= 1 && j - 1 <= jmax) pv((j - 1) % NV, Pprev);
     __builtin_amdgcn_sched_barrier(0);
     if (j <= jmax) {
       if (j < nfull) softmax(j, Pcur, false);
       else softmax(j, Pcur, true);
       keep_p();
     }
-    if (j + 1 <= jmax) qk(j + 1, (j + 1) % NBUF);
-    sync_tiles(j + 3 < nkb);
+    if (j + 1 <= jmax) qk(j + 1, (j + 1) % NK);
+    sync_tiles(j + 3 < nkb, j + kVA < nkb);
   };
   // blocks 1 <= j < j_fast: every stage exists and no mask is needed; the P.V
   // MFMAs of block j-1 and the softmax VALU work of block j share one basic
   // block for the scheduler to interleave
-  // sl: j % NBUF as a constant (the unrolled loop: operand offsets fold into
-  // the LDS instructions), or -1 to compute the slots from j
+  // sl: j % NK == j % NV as a constant (the unrolled loop: operand offsets
+  // fold into the LDS instructions), or -1 to compute the slots from j
+  auto fast_loads = [&](int j, int sl) __attribute__((always_inline)) {
+    load_v(j + kVA, sl < 0 ? (j + kVA) % NV : (sl + kVA) % NV);
+    load_k(j + 3, sl < 0 ? (j + 3) % NK : (sl + 3) % NK, true);
+  };
   auto fast_iter = [&](int j, int sl) __attribute__((always_inline)) {
-    load_tile_fast(j + 3, sl < 0 ? (j + 3) % NBUF : (sl + 3) % NBUF);
+    fast_loads(j, sl);
     if (pend) {
       rescale_o();
       pend = false;
     }
-    pv(sl < 0 ? (j - 1) % NBUF : (sl + NBUF - 1) % NBUF, Pprev);
+    pv(sl < 0 ? (j - 1) % NV : (sl + NV - 1) % NV, Pprev);
     __builtin_amdgcn_iglp_opt(0);  // LLVM's IGroupLP strategy 0, as in fused_iter below
     if constexpr (PVM != SAGE_PV_FP8) softmax_fast(j, Pcur);
     else softmax(j, Pcur, false);
     keep_p();
-    qk(j + 1, sl < 0 ? (j + 1) % NBUF : (sl + 1) % NBUF);
-    sync_tiles(true, true);
+    qk(j + 1, sl < 0 ? (j + 1) % NK : (sl + 1) % NK);
+    sync_tiles(true, true, true);
   };
 
   // INT8 with fp16 P, and fp16/bf16 QK at D = 64: the S of block j+1 goes to
@@ -822,20 +840,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float ksc2 = 0.0f;
   auto fused_iter = [&](int j, int sl, SAcc (&Sa)[2], float ka, SAcc (&Sb)[2], float& kb)
                         __attribute__((always_inline)) {
-    load_tile_fast(j + 3, sl < 0 ? (j + 3) % NBUF : (sl + 3) % NBUF);
+    fast_loads(j, sl);
     if (pend) {
       rescale_o();
       pend = false;
     }
-    pv(sl < 0 ? (j - 1) % NBUF : (sl + NBUF - 1) % NBUF, Pprev);
+    pv(sl < 0 ? (j - 1) % NV : (sl + NV - 1) % NV, Pprev);
     // LLVM's IGroupLP strategy 0 (LDS instructions interleaved with MFMAs)
     // for this scheduling region: measured -1.5 to -2 % per attention launch at
     // configs 2 and 3, -3 % at config 4, +-0 at config 5
     __builtin_amdgcn_iglp_opt(0);
-    qk_into(j + 1, sl < 0 ? (j + 1) % NBUF : (sl + 1) % NBUF, Sb, kb);
+    qk_into(j + 1, sl < 0 ? (j + 1) % NK : (sl + 1) % NK, Sb, kb);
     softmax_fast_on(j, Pcur, Sa, ka);
     keep_p();
-    sync_tiles(true, true);
+    sync_tiles(true, true, true);
   };
 
   // Q quantization (kFQ) with the pre-pass's arithmetic (per_block_int8,
@@ -846,7 +864,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto quantize_q = [&]() __attribute__((always_inline)) {
     if constexpr (kFQ) {
 #pragma clang fp contract(off)
-      __shared__ float qamax_s[NW];
+      float* qamax_s = reinterpret_cast<float*>(smem + RING + SINK);
       const int row = qa + n;
       const bool valid = row < a.Nq;
       float xq[KC][16];
@@ -905,22 +923,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   };
 
-  // ---- prologue: tiles 0, 1, 2 requested, 0 and 1 awaited; S of block 0.
-  // With fewer than 3 tiles the last one is requested again (same data into
-  // its own slot), so the number of loads issued after Q's is fixed and Q can
-  // be waited for without draining the tile loads.
-  load_tile(0, 0);
-  load_tile(min(1, nkb - 1), min(1, nkb - 1));
-  load_tile(min(2, nkb - 1), min(2, nkb - 1));
+  // ---- prologue: K tiles 0, 1, 2 (and V tile 0) requested, K 0 and 1
+  // awaited; S of block 0.  With fewer than 3 tiles the last one is requested
+  // again (same data into its own slot), so the number of loads issued after
+  // Q's is fixed and Q can be waited for without draining the tile loads.
+  load_k(0, 0, false);
+  load_k(min(1, nkb - 1), min(1, nkb - 1), false);
+  if constexpr (kVA > 0) load_v(0, 0);
+  load_k(min(2, nkb - 1), min(2, nkb - 1), false);
   quantize_q();
 #if SAGE_TRACE
   tr_put(13, __builtin_amdgcn_s_memtime());
 #endif
-  sync_tiles(nkb > 2);
+  sync_tiles(true, true);
 #if SAGE_TRACE
   tr_put(14, __builtin_amdgcn_s_memtime());
 #endif
   if (jmax >= 0) qk(0, 0);
+  if constexpr (NK == 3) {  // iteration 0 loads K tile 3 into the slot just read
+    SAGE_WAIT_LGKM0();
+    wg_barrier();
+  }
 
   if constexpr (kI8) {  // mgrid = 4 ulp(kMagicF * c_max): exponent field of that product - 21,
     // at least 2^-23 (a coarser grid keeps the bias exact; with a zero scale
@@ -940,29 +963,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   tr_put(2, __builtin_amdgcn_s_memtime());
 #endif
   int j = 1;
-  // D = 64 (INT8 with fp16 P, and fp16/bf16 QK): constant ring slots, j % NBUF
-  // == 1 at every trip (at D = 128 the copies run out of registers); then
-  // INT8 with fp16 P five at a time with one S buffer
+  // D = 64: constant ring slots, j % 4 == 1 at every trip (at D = 128 the
+  // copies run out of registers); the two S buffers swap every iteration
+  static_assert(D != 64 || (NK == 4 && NV == 4), "unrolled by the ring");
   if constexpr (kTwoS && D == 64)
-    for (; j + 2 * NBUF <= j_fast; j += 2 * NBUF) {
+    for (; j + 4 <= j_fast; j += 4) {
       fused_iter(j, 1, S, ksc_cur, S2, ksc2);
       fused_iter(j + 1, 2, S2, ksc2, S, ksc_cur);
       fused_iter(j + 2, 3, S, ksc_cur, S2, ksc2);
-      fused_iter(j + 3, 4, S2, ksc2, S, ksc_cur);
-      fused_iter(j + 4, 0, S, ksc_cur, S2, ksc2);
-      fused_iter(j + 5, 1, S2, ksc2, S, ksc_cur);
-      fused_iter(j + 6, 2, S, ksc_cur, S2, ksc2);
-      fused_iter(j + 7, 3, S2, ksc2, S, ksc_cur);
-      fused_iter(j + 8, 4, S, ksc_cur, S2, ksc2);
-      fused_iter(j + 9, 0, S2, ksc2, S, ksc_cur);
-    }
-  if constexpr (kI8 && D == 64 && PVM == SAGE_PV_F16)
-    for (; j + NBUF <= j_fast; j += NBUF) {
-      fast_iter(j, 1);
-      fast_iter(j + 1, 2);
-      fast_iter(j + 2, 3);
-      fast_iter(j + 3, 4);
-      fast_iter(j + 4, 0);
+      fused_iter(j + 3, 0, S2, ksc2, S, ksc_cur);
     }
   if constexpr (kTwoS && D == 128)
     for (; j + 2 <= j_fast; j += 2) {
@@ -1000,7 +1009,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // with LDS reads and tile loads drained and a barrier) tile ring, it goes
   // through LDS and leaves as whole rows, 16 bytes per lane.
   constexpr int ORP = D * (int)sizeof(TO) + 16;  // LDS row pitch: rows 4 banks apart
-  if constexpr (NW * 32 * ORP <= NBUF * SLOT) {
+  if constexpr (NW * 32 * ORP <= RING) {
     char* st = smem + wave * 32 * ORP;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -1046,18 +1055,19 @@ static int64_t g_trace_words = 0;
 
 template <int QKM, int D, int PVM, typename TO>
 static int launch_cfg(const AttnArgs& a, hipStream_t st, const char* who) {
-  const int64_t nqb = (a.Nq + 255) / 256;
+  constexpr int NW = 8;
+  const int64_t nqb = (a.Nq + 32 * NW - 1) / (32 * NW);
   const int64_t grid = nqb * a.Hq * a.B;
   if (grid > 0x7FFFFFFF) return fail("%s: invalid argument: grid too large", who);
 #if SAGE_TRACE
   AttnArgs at = a;
   at.trace = g_trace;
-  if (g_trace && grid * 8 * kTraceWords > g_trace_words)
+  if (g_trace && grid * NW * kTraceWords > g_trace_words)
     return fail("%s: invalid argument: trace buffer of %lld words < %lld", who, (long long)g_trace_words,
-                (long long)(grid * 8 * kTraceWords));
-  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO>), dim3((unsigned)grid), dim3(512), 0, st, at);
+                (long long)(grid * NW * kTraceWords));
+  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW>), dim3((unsigned)grid), dim3(64 * NW), 0, st, at);
 #else
-  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO>), dim3((unsigned)grid), dim3(512), 0, st, a);
+  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW>), dim3((unsigned)grid), dim3(64 * NW), 0, st, a);
 #endif
   return check_launch(who);
 }
