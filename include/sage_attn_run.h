@@ -1,0 +1,47 @@
+/*
+ * sage_attn_run.h — whole-call entry points of libsage_attn.so.
+ *
+ * sage_attn.h offers the stages (pre-pass, V tiles, attention) one by one;
+ * the calls here take a user's Q, K, V and O and choose the stages, kernels
+ * and launch shapes themselves.  They share its conventions: strides are the
+ * element strides of batch, head and sequence, rows are 16-byte aligned, the
+ * caller owns every buffer, calls are asynchronous on `stream`, a non-zero
+ * status leaves a message in sage_last_error().
+ *
+ *   sage_flash_run() <- run_flash_attn (kernels/flash_attn/triton_impl.py:103-121)
+ */
+#ifndef SAGE_ATTN_RUN_H
+#define SAGE_ATTN_RUN_H
+
+#include <stddef.h>
+#include <stdint.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* One call.  Every field is 8 bytes, so a binding can pack it as an array. */
+typedef struct sage_call {
+  int64_t size; /* sizeof(sage_call): a caller built for another layout is refused */
+  const void* q;
+  const void* k;
+  const void* v;
+  void* o; /* [B,Hq,Nq,D] in dtype */
+  int64_t q_strides[3], k_strides[3], v_strides[3], o_strides[3];
+  int64_t B, Hq, Hkv, Nq, Nkv, D;
+  double mul;     /* fp32(sm_scale * 1.44269504): scores in log2 units */
+  int64_t dtype;  /* of q, k, v and o: SAGE_DTYPE_* */
+  int64_t causal; /* 1: key j is visible to query i iff j <= i */
+} sage_call;
+
+/*
+ * Unquantized attention on fp16 / bf16 inputs: sage_flash_fwd with V read
+ * where it is (no V tiles).  Row strides of V must be below 2^25 elements.
+ */
+int sage_flash_run(const sage_call* call, void* stream);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif /* SAGE_ATTN_RUN_H */

@@ -1,0 +1,71 @@
+"""V read in place by the unquantized kernel (sage_flash_run) against the V tile path.
+
+Both run the same arithmetic in the same order on the same V bits, so the
+outputs are equal bit for bit: at lengths around the 64-key tile (one key, a
+tail of one, whole tiles, the mask-free loop with and without leftovers), for
+both types and head dims, causal and not, and with V rows that are slices of
+wider rows.  V rows too far apart for the in-place loads take the tile path.
+"""
+from __future__ import annotations
+
+import ctypes
+import importlib.util
+from pathlib import Path
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+FLASH = Path(__file__).resolve().parents[1] / "tribench_amd" / "kernels" / "flash_attn" / "hip_impl.py"
+
+
+def _flash():
+    spec = importlib.util.spec_from_file_location("flash_vrow_impl", FLASH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+def _tiles(H, q, k, v, causal, layout="HND"):
+    """sage_vtiles + sage_flash_fwd, stage by stage."""
+    lib = H._load()
+    B, Hq, Hkv, Nq, Nkv, D = H._check_inputs(q, k, v, layout)
+    vt = H.vtiles(v, {torch.float16: "fp16", torch.bfloat16: "bf16"}[q.dtype], tensor_layout=layout)
+    o = torch.empty_like(q)
+    mul = ctypes.c_float(float(np.float32(D ** -0.5 * H.LOG2E_REF)))
+    rc = lib.sage_flash_fwd(H._ptr(q), H._strides(q, layout), H._ptr(k), H._strides(k, layout), H._ptr(vt),
+                            H.DTYPE_VTILES, None, H._ptr(o), H._strides(o, layout), H._TORCH_CODES[q.dtype],
+                            B, Hq, Hkv, Nq, Nkv, D, mul, int(causal), H._stream(q.device))
+    H._check(rc, "sage_flash_fwd")
+    return o
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Nq,Nkv,causal", [(1, 1, False), (5, 63, False), (65, 65, True), (129, 128, False),
+                                           (300, 257, False), (448, 448, True), (33, 705, False)])
+def test_in_place_equals_tiles(D, dtype, Nq, Nkv, causal, gpu_device):
+    print(f"[vrow] D{D} {dtype} {Nq}/{Nkv} causal={causal}", flush=True)
+    F = _flash()
+    g = torch.Generator().manual_seed(Nq * 1000 + Nkv)
+    q = torch.randn(2, 4, Nq, D, generator=g).to(dtype).to(gpu_device)
+    k = torch.randn(2, 2, Nkv, D, generator=g).to(dtype).to(gpu_device)
+    wide = torch.randn(2, Nkv, 2, D + 8, generator=g).to(dtype).to(gpu_device)  # sequence-major, padded rows
+    v = wide[..., :D].transpose(1, 2)
+    got = F.run(q, k, v, causal=causal)
+    torch.cuda.synchronize()
+    assert torch.equal(got, _tiles(F._H, q, k, v, causal))
+    nhd = [t.transpose(1, 2).contiguous() for t in (q, k, v)]
+    got = F.run(*nhd, causal=causal, tensor_layout="NHD")
+    assert torch.equal(got, _tiles(F._H, *nhd, causal, "NHD"))
+
+
+def test_far_apart_rows_take_the_tile_path(gpu_device):
+    F = _flash()
+    base = torch.randn((1 << 25) + 64, device=gpu_device, dtype=torch.float16)
+    v = base.as_strided((1, 1, 2, 64), (0, 0, 1 << 25, 1))
+    q, k = (torch.randn(1, 1, 2, 64, device=gpu_device, dtype=torch.float16) for _ in range(2))
+    got = F.run(q, k, v)
+    torch.cuda.synchronize()
+    assert torch.equal(got, F.run(q, k, v.contiguous()))

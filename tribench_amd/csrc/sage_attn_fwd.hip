@@ -20,9 +20,10 @@
 //    (fp32, 32 x D) all live in arch VGPRs.
 //  * K8 rows and V^T rows reach LDS in tiles of 64 keys by direct global ->
 //    LDS loads (global_load_lds_dwordx4), two iterations ahead of their use, in
-//    a ring of K tiles and one of V tiles: no staging registers, no VALU work.  V arrives
-//    already converted and transposed (sage_vtiles), so a tile is a plain
-//    copy.  The 16-byte chunks of each LDS row are XOR-swizzled so that the
+//    a ring of K tiles and one of V tiles: no staging registers, no VALU work.
+//    V arrives already converted and transposed (sage_vtiles), so a tile is a
+//    plain copy; the unquantized kernel also takes V as it is (kVRow) and
+//    transposes in the operand read.  The 16-byte chunks of each LDS row are XOR-swizzled so that the
 //    operand reads of 16 consecutive lanes (rows) hit distinct banks.
 //  * Each wave waits (vmcnt) for exactly its own loads of the tile the next
 //    iteration reads, then meets the others at a barrier without a memory
@@ -49,6 +50,7 @@
 #include <type_traits>
 
 #include "sage_device.h"
+#include "../../include/sage_attn_run.h"
 
 // SAGE_TRACE (a measurement build only, libsage_attn_trace.so): every wave
 // records s_memtime at its phase boundaries and the cycles it spends at the
@@ -68,11 +70,13 @@ struct AttnArgs {
   const float* q_scale;
   const void* k8;         // INT8 K (or fp16/bf16 K)
   const float* k_scale;
-  const void* v;          // V tiles (sage_vtiles layout)
+  const void* v;          // V tiles (sage_vtiles layout), or V itself (kVRow)
   const float* v_scale;
   void* o;
   int64_t sq[2], sk[2], so[2];  // batch and head strides (elements)
   int sqn, skn, son;            // row strides (elements); row offsets fit 32 bits
+  int64_t sv[2];                // V read in place: batch and head strides, row stride
+  int svn, vrow;
   int B, Hq, Hkv, Nq, Nkv;
   int causal;
   int q_sub, blkk_shift;  // k scale of key block j: k_scale[j >> blkk_shift]
@@ -253,6 +257,23 @@ __device__ __forceinline__ int swz(int r) {
 
 typedef __attribute__((address_space(1))) const void gmem_t;
 typedef __attribute__((address_space(3))) void lmem_t;
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4s ltr_t;
+
+__device__ __forceinline__ v4i lds_read16(const char* p) { return *reinterpret_cast<const v4i*>(p); }
+// (an alias scope of its own, from __restrict__: without it the compiler
+// drains every direct-to-LDS load in flight before the read)
+__device__ __forceinline__ v2i lds_read_tr(const char* __restrict__ p) {
+  return __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ltr_t*)p));
+}
+
+// swz() for rows of V read in place (2*D bytes, read 4 rows x 32 bytes at
+// a time by 16 lanes): 64-byte quarters rotate with the row, so that 4
+// consecutive rows of one 64-byte column cover all 64 banks.
+template <int D>
+__device__ __forceinline__ int vrow_swz(int r) {
+  return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1);
+}
 
 // LDS rings of the tile loads.  Iteration j reads K tile j+1 and V tile j-1
 // while K tiles j+2, j+3 and V tiles j .. j+kVA arrive: at least 3 K slots and
@@ -275,7 +296,7 @@ struct TileRing {
 // each) of one (batch, head); Q rows, S, P and the O^T accumulators live in
 // arch VGPRs.  Tiles of 64 keys (K rows and V^T rows) reach LDS by direct
 // global -> LDS loads, two iterations ahead of their use (TileRing).
-template <int QKM, int D, int PVM, typename TO, int NW>
+template <int QKM, int D, int PVM, typename TO, int NW, bool kVRow>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_kernel(AttnArgs a) {
   constexpr int BM = 32 * NW;  // query rows per work-group
   constexpr bool kFQ = QKM == kQkI8Q;  // Q quantized in the prologue
@@ -303,6 +324,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   constexpr int LPW = KPW + VPW;
   static_assert(LPW <= 15, "tile loads");
   constexpr int SINK = KPW * NW > KLD || VPW * NW > VLD ? 1024 : 0;  // target of spare loads
+  static_assert(!kVRow || EB == 2, "V is read in place in a 16-bit type");
 
   // One LDS array for everything: with a second __shared__ variable the
   // compiler gives LDS accesses alias scopes, takes the operand reads of the
@@ -361,7 +383,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   typedef __attribute__((address_space(4))) const float cfloat_t;
   cfloat_t* ksc_base = (cfloat_t*)(a.k_scale + ((int64_t)b * a.Hkv + hk) * a.nks);
   const int ntile = (a.Nkv + kBN - 1) / kBN;
-  const uint8_t* vtbase = static_cast<const uint8_t*>(a.v) + ((int64_t)b * a.Hkv + hk) * ntile * (int64_t)VTB;
+  const uint8_t* vtbase = static_cast<const uint8_t*>(a.v);
+  if constexpr (kVRow) vtbase += (b * a.sv[0] + hk * a.sv[1]) * EB;
+  else vtbase += ((int64_t)b * a.Hkv + hk) * ntile * (int64_t)VTB;
 
   // ---- the largest k scale of the head (INT8), for the grid of the running
   // max below; loaded before every other load, so that waiting for it waits
@@ -417,8 +441,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   // ---- tile loads.  Wave load g = wave + NW*i of a K (V) tile is the 1 KB LDS
   // range [1024g, 1024g + 1024) of its slot; lane l brings the 16-byte chunk
   // that lands at offset 16l, i.e. the logical chunk (physical chunk ^ swizzle
-  // of its row).  K rows past Nkv read the last row (their P is 0); V tiles
-  // are zero past Nkv.  Loads past the tile go to the sink, so every
+  // of its row).  K rows past Nkv read the last row (their P is 0), rows of V
+  // read in place too (P = 0 meets a value that the block holds anyway); V
+  // tiles are zero past Nkv.  Loads past the tile go to the sink, so every
   // wave issues KPW loads per K tile and VPW per V tile.  `whole`: every row
   // of the tile is < Nkv, so each load is a uniform tile base plus a lane
   // offset that does not change from tile to tile.
@@ -432,10 +457,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
   for (int i = 0; i < VPW; ++i) {
     const int p = 64 * (wave + NW * i) + lane;
-    const int d = p / (VRB / 16), pc = p % (VRB / 16);
-    vfoff[i] = wave + NW * i < VLD ? (uint32_t)(d * VRB + 16 * (pc ^ swz<VRB>(d))) : 0u;
+    if constexpr (kVRow) {
+      const int r = p / (2 * D / 16), pc = p % (2 * D / 16);
+      vfoff[i] = wave + NW * i < VLD ? (uint32_t)(r * a.svn * EB + 16 * (pc ^ vrow_swz<D>(r))) : 0u;
+    } else {
+      const int d = p / (VRB / 16), pc = p % (VRB / 16);
+      vfoff[i] = wave + NW * i < VLD ? (uint32_t)(d * VRB + 16 * (pc ^ swz<VRB>(d))) : 0u;
+    }
   }
   const int64_t ktile_bytes = (int64_t)kBN * a.skn * QEB;
+  const int64_t vtile_bytes = kVRow ? (int64_t)kBN * a.svn * EB : (int64_t)VTB;
   auto load_k = [&](int j, int sl, bool whole) __attribute__((always_inline)) {  // sl = j % NK
     char* slot = smem + sl * KTB;
     const char* base = kbase + j * ktile_bytes;
@@ -455,15 +486,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
       __builtin_amdgcn_global_load_lds((gmem_t*)src, (lmem_t*)dst, 16, 0, 0);
     }
   };
-  auto load_v = [&](int j, int sl) __attribute__((always_inline)) {  // sl = j % NV
+  auto load_v = [&](int j, int sl, bool whole) __attribute__((always_inline)) {  // sl = j % NV
     char* slot = smem + VOFF + sl * VTB;
-    const char* base = reinterpret_cast<const char*>(vtbase) + (int64_t)j * VTB;
+    const char* base = reinterpret_cast<const char*>(vtbase) + j * vtile_bytes;
     asm("" : "+s"(base));
 #pragma unroll
     for (int i = 0; i < VPW; ++i) {
       const int g = wave + NW * i;  // wave-uniform
       const bool in = VLD % NW == 0 || g < VLD;
       const char* src = in ? base + vfoff[i] : kbase;
+      if (kVRow && !whole && in) {
+        const int p = 64 * g + lane;
+        const int r = p / (2 * D / 16), pc = p % (2 * D / 16);
+        src = base + (uint32_t)(min(r, a.Nkv - 1 - j * kBN) * a.svn * EB + 16 * (pc ^ vrow_swz<D>(r)));
+      }
       char* dst = in ? slot + 1024 * g : smem + RING;
       __builtin_amdgcn_global_load_lds((gmem_t*)src, (lmem_t*)dst, 16, 0, 0);
     }
@@ -542,6 +578,24 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   int voff[VCH];  // V^T row 32dt + n (swizzle independent of dt)
 #pragma unroll
   for (int c = 0; c < VCH; ++c) voff[c] = VOFF + n * VRB + 16 * ((VCH * hh + c) ^ swz<VRB>(n));
+  // V in place (no V tile pass: one launch and 4 bytes of traffic per element
+  // less, 42 us at B4 H32 N4096 D128; the operand takes two 8-byte reads in
+  // place of one of 16, so the loop itself is no faster): whole calls 1029 ->
+  // 968 us there, 167 -> 140 us for one query row over 8192 keys (B8, 8 KV
+  // heads), 27 -> 15 us at B1 H16 N512 D64.  ds_read_b64_tr_b16 hands lane i of each 16 lanes column i of
+  // the 4 rows that its lanes address (4 lanes to a row of 16 elements), so
+  // lane (hh, n) gets channel 32dt + n of keys 32t + 8i + 4hh .. +4 when its
+  // 16 lanes address those keys.  The rows of a 4-key group sit in different
+  // 64-byte quarters of the banks (vrow_swz).
+  int vtoff[kVRow ? DT : 1];
+  if constexpr (kVRow) {
+    const int r = (lane & 15) >> 2;  // row of the group; key = 4hh + r of each 8
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const int c = 4 * dt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);  // 16-byte chunk of the row
+      vtoff[dt] = VOFF + (4 * hh + r) * 2 * D + 16 * (c ^ vrow_swz<D>(r)) + 8 * (lane & 1);
+    }
+  }
 
   // ---- building blocks
   // S^T of block j (its K tile in slot j % NK): K row 32t + n, bytes 32c + 16hh
@@ -555,7 +609,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     for (int t = 0; t < 2; ++t) {
       v4i ka[KC];
 #pragma unroll
-      for (int c = 0; c < KC; ++c) ka[c] = *reinterpret_cast<const v4i*>(ks + 32 * t * KRB + koff[c]);
+      for (int c = 0; c < KC; ++c) ka[c] = lds_read16(ks + 32 * t * KRB + koff[c]);
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
         if constexpr (kI8) {
@@ -581,8 +635,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     for (int dt = 0; dt < DT; ++dt) {
       const char* vr = vs + 32 * dt * VRB;
       if constexpr (kF8) {
-        const v4i lo = *reinterpret_cast<const v4i*>(vr + voff[0]);
-        const v4i hi = *reinterpret_cast<const v4i*>(vr + voff[1]);
+        const v4i lo = lds_read16(vr + voff[0]);
+        const v4i hi = lds_read16(vr + voff[1]);
         const v8i va = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         const v8i pb = {(int)P[0], (int)P[1], (int)P[2], (int)P[3], (int)P[4], (int)P[5], (int)P[6], (int)P[7]};
         oacc[dt] = Pv::mma(va, pb, oacc[dt]);
@@ -591,7 +645,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
       } else {
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {  // 16-key steps: key tile kk/2, register half kk%2
-          const v4i va = *reinterpret_cast<const v4i*>(vr + voff[kk]);
+          v4i va;
+          if constexpr (kVRow) {  // keys 16kk + 4hh .. +4 and 8 further on
+            const char* vk = vs + vtoff[dt] + 16 * kk * 2 * D;
+            const v2i lo = lds_read_tr(vk);
+            const v2i hi = lds_read_tr(vk + 8 * 2 * D);
+            va = (v4i){lo.x, lo.y, hi.x, hi.y};
+          } else {
+            va = lds_read16(vr + voff[kk]);
+          }
           const v4i pb = {(int)P[4 * kk], (int)P[4 * kk + 1], (int)P[4 * kk + 2], (int)P[4 * kk + 3]};
           oacc[dt] = Pv::mma(va, pb, oacc[dt]);
         }
@@ -786,7 +848,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   // iterations.  The mask-free steady state has a loop of its own so that the
   // O accumulators are updated from one place in each loop.
   auto generic_iter = [&](int j) __attribute__((always_inline)) {
-    if (j + kVA < nkb) load_v(j + kVA, (j + kVA) % NV);
+    if (j + kVA < nkb) load_v(j + kVA, (j + kVA) % NV, false);
     if (j + 3 < nkb) load_k(j + 3, (j + 3) % NK, false);
     if (pend) {
       rescale_o();
@@ -808,7 +870,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   // sl: j % NK == j % NV as a constant (the unrolled loop: operand offsets
   // fold into the LDS instructions), or -1 to compute the slots from j
   auto fast_loads = [&](int j, int sl) __attribute__((always_inline)) {
-    load_v(j + kVA, sl < 0 ? (j + kVA) % NV : (sl + kVA) % NV);
+    load_v(j + kVA, sl < 0 ? (j + kVA) % NV : (sl + kVA) % NV, true);
     load_k(j + 3, sl < 0 ? (j + 3) % NK : (sl + 3) % NK, true);
   };
   auto fast_iter = [&](int j, int sl) __attribute__((always_inline)) {
@@ -929,7 +991,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   // Q's is fixed and Q can be waited for without draining the tile loads.
   load_k(0, 0, false);
   load_k(min(1, nkb - 1), min(1, nkb - 1), false);
-  if constexpr (kVA > 0) load_v(0, 0);
+  if constexpr (kVA > 0) load_v(0, 0, false);
   load_k(min(2, nkb - 1), min(2, nkb - 1), false);
   quantize_q();
 #if SAGE_TRACE
@@ -1053,9 +1115,8 @@ static unsigned long long* g_trace = nullptr;
 static int64_t g_trace_words = 0;
 #endif
 
-template <int QKM, int D, int PVM, typename TO>
-static int launch_cfg(const AttnArgs& a, hipStream_t st, const char* who) {
-  constexpr int NW = 8;
+template <int QKM, int D, int PVM, typename TO, int NW, bool kVRow>
+static int launch_nw(const AttnArgs& a, hipStream_t st, const char* who) {
   const int64_t nqb = (a.Nq + 32 * NW - 1) / (32 * NW);
   const int64_t grid = nqb * a.Hq * a.B;
   if (grid > 0x7FFFFFFF) return fail("%s: invalid argument: grid too large", who);
@@ -1065,11 +1126,19 @@ static int launch_cfg(const AttnArgs& a, hipStream_t st, const char* who) {
   if (g_trace && grid * NW * kTraceWords > g_trace_words)
     return fail("%s: invalid argument: trace buffer of %lld words < %lld", who, (long long)g_trace_words,
                 (long long)(grid * NW * kTraceWords));
-  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW>), dim3((unsigned)grid), dim3(64 * NW), 0, st, at);
+  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW, kVRow>), dim3((unsigned)grid), dim3(64 * NW), 0, st, at);
 #else
-  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW>), dim3((unsigned)grid), dim3(64 * NW), 0, st, a);
+  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW, kVRow>), dim3((unsigned)grid), dim3(64 * NW), 0, st, a);
 #endif
   return check_launch(who);
+}
+
+template <int QKM, int D, int PVM, typename TO>
+static int launch_cfg(const AttnArgs& a, hipStream_t st, const char* who) {
+  constexpr int NW = 8;
+  if constexpr (QKM == kQkF16 || QKM == kQkBF16)
+    if (a.vrow) return launch_nw<QKM, D, PVM, TO, NW, true>(a, st, who);
+  return launch_nw<QKM, D, PVM, TO, NW, false>(a, st, who);
 }
 
 template <int PVM, typename TO>
@@ -1251,37 +1320,30 @@ extern "C" int sage_trace_attach(unsigned long long* buf, int64_t words) {
 }
 #endif
 
-extern "C" int sage_flash_fwd(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
-                              const void* v, int v_dtype, const int64_t* v_strides, void* o,
-                              const int64_t* o_strides, int in_dtype, int64_t B, int64_t Hq, int64_t Hkv,
-                              int64_t Nq, int64_t Nkv, int64_t D, float qk_mul, int causal, void* stream) {
-  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Nq <= 0 || Nkv <= 0)
-    return fail("sage_flash_fwd: invalid argument: empty shape");
+// Checks of the unquantized kernel and everything of AttnArgs but V.
+static int flash_setup(AttnArgs& a, const char* who, const void* q, const int64_t* q_strides, const void* k,
+                       const int64_t* k_strides, void* o, const int64_t* o_strides, int in_dtype, int64_t B,
+                       int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nkv, int64_t D, float qk_mul, int causal) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Nq <= 0 || Nkv <= 0) return fail("%s: invalid argument: empty shape", who);
   if (D != 64 && D != 128)
-    return fail("sage_flash_fwd: invalid argument: head_dim %lld (supported: 64, 128)", (long long)D);
-  if (Hq % Hkv != 0) return fail("sage_flash_fwd: invalid argument: Hq %% Hkv != 0");
+    return fail("%s: invalid argument: head_dim %lld (supported: 64, 128)", who, (long long)D);
+  if (Hq % Hkv != 0) return fail("%s: invalid argument: Hq %% Hkv != 0", who);
   if (Nq > 0x7FFFFFFF || Nkv > 0x7FFFFFFF || Hq > 0xFFFF || B > 0xFFFF)
-    return fail("sage_flash_fwd: invalid argument: shape too large");
+    return fail("%s: invalid argument: shape too large", who);
   if (in_dtype != SAGE_DTYPE_F16 && in_dtype != SAGE_DTYPE_BF16)
-    return fail("sage_flash_fwd: invalid argument: in_dtype %d (fp16 or bf16)", in_dtype);
-  if (!q || !k || !v || !o || !q_strides || !k_strides || !o_strides)
-    return fail("sage_flash_fwd: invalid argument: null pointer");
-  if (v_dtype != SAGE_DTYPE_VTILES)
-    return fail("sage_flash_fwd: invalid argument: v_dtype %d (V must be in the tile layout of sage_vtiles)",
-                v_dtype);
-  if (!(qk_mul > 0.0f) || qk_mul == INFINITY) return fail("sage_flash_fwd: invalid argument: qk_mul %g", qk_mul);
+    return fail("%s: invalid argument: in_dtype %d (fp16 or bf16)", who, in_dtype);
+  if (!q || !k || !o || !q_strides || !k_strides || !o_strides)
+    return fail("%s: invalid argument: null pointer", who);
+  if (!(qk_mul > 0.0f) || qk_mul == INFINITY) return fail("%s: invalid argument: qk_mul %g", who, qk_mul);
   const bool rows32 = (Nq * q_strides[2] + D) * 2 < 0x7FFFFFFF && (Nkv * k_strides[2] + D) * 2 < 0x7FFFFFFF &&
                       Nq * o_strides[2] + D < 0x7FFFFFFF;
-  if (!rows32) return fail("sage_flash_fwd: invalid argument: a head's rows must span < 2^31 bytes");
+  if (!rows32) return fail("%s: invalid argument: a head's rows must span < 2^31 bytes", who);
   if (!strides_ok(q_strides, 2) || !strides_ok(k_strides, 2) || !strides_ok(o_strides, 2))
-    return fail("sage_flash_fwd: invalid argument: strides must keep 16-byte aligned rows");
-  if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) % 16 != 0)
-    return fail("sage_flash_fwd: invalid argument: base pointers must be 16-byte aligned");
-
-  AttnArgs a{};
+    return fail("%s: invalid argument: strides must keep 16-byte aligned rows", who);
+  if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)o) % 16 != 0)
+    return fail("%s: invalid argument: base pointers must be 16-byte aligned", who);
   a.q8 = q;
   a.k8 = k;
-  a.v = v;
   a.o = o;
   for (int i = 0; i < 2; ++i) {
     a.sq[i] = q_strides[i];
@@ -1300,8 +1362,44 @@ extern "C" int sage_flash_fwd(const void* q, const int64_t* q_strides, const voi
   a.q_sub = 32;
   a.nqs = a.nks = 1;
   a.qk_mul = qk_mul;
+  return 0;
+}
+
+extern "C" int sage_flash_fwd(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                              const void* v, int v_dtype, const int64_t* v_strides, void* o,
+                              const int64_t* o_strides, int in_dtype, int64_t B, int64_t Hq, int64_t Hkv,
+                              int64_t Nq, int64_t Nkv, int64_t D, float qk_mul, int causal, void* stream) {
+  (void)v_strides;
+  const char* who = "sage_flash_fwd";
+  AttnArgs a{};
+  if (int rc = flash_setup(a, who, q, q_strides, k, k_strides, o, o_strides, in_dtype, B, Hq, Hkv, Nq, Nkv, D,
+                           qk_mul, causal))
+    return rc;
+  if (!v) return fail("%s: invalid argument: null pointer", who);
+  if (v_dtype != SAGE_DTYPE_VTILES)
+    return fail("%s: invalid argument: v_dtype %d (V must be in the tile layout of sage_vtiles)", who, v_dtype);
+  if ((uintptr_t)v % 16 != 0) return fail("%s: invalid argument: base pointers must be 16-byte aligned", who);
+  a.v = v;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int d = (int)D;
-  return in_dtype == SAGE_DTYPE_F16 ? launch_flash<kQkF16, _Float16>(a, d, st)
-                                    : launch_flash<kQkBF16, __bf16>(a, d, st);
+  return in_dtype == SAGE_DTYPE_F16 ? launch_flash<kQkF16, _Float16>(a, (int)D, st)
+                                    : launch_flash<kQkBF16, __bf16>(a, (int)D, st);
+}
+
+extern "C" int sage_flash_run(const sage_call* c, void* stream) {
+  const char* who = "sage_flash_run";
+  if (!c || c->size != (int64_t)sizeof(sage_call)) return fail("%s: invalid argument: sage_call size", who);
+  AttnArgs a{};
+  if (int rc = flash_setup(a, who, c->q, c->q_strides, c->k, c->k_strides, c->o, c->o_strides, (int)c->dtype, c->B,
+                           c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, (float)c->mul, (int)c->causal))
+    return rc;
+  if (!c->v || (uintptr_t)c->v % 16 != 0 || !strides_ok(c->v_strides, 2) || c->v_strides[2] >= (1 << 25))
+    return fail("%s: invalid argument: V must have 16-byte aligned rows less than 2^25 elements apart", who);
+  a.v = c->v;
+  a.sv[0] = c->v_strides[0];
+  a.sv[1] = c->v_strides[1];
+  a.svn = (int)c->v_strides[2];
+  a.vrow = 1;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return c->dtype == SAGE_DTYPE_F16 ? launch_flash<kQkF16, _Float16>(a, (int)c->D, st)
+                                    : launch_flash<kQkBF16, __bf16>(a, (int)c->D, st);
 }

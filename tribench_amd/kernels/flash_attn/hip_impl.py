@@ -2,11 +2,11 @@
 
 ``run`` has the call signature of ``run_flash_attn`` (kernels/flash_attn/
 triton_impl.py:103) and is registered as ``variants: {"hip": "hip_impl.py:run"}``.
-It runs the attention kernel of libsage_attn.so on unquantized fp16/bf16 Q
-and K (C-ABI ``sage_flash_fwd``): S = Q K^T in fp32 from fp16/bf16 MFMAs, an
-online softmax, P rounded to V's dtype as the reference does (:87-88), P.V
-accumulated in fp32.  V first goes through ``sage_vtiles`` (the 16-bit V^T
-tile layout the kernel copies into LDS).
+It runs the attention kernel of libsage_attn.so on unquantized fp16/bf16 Q,
+K and V (C-ABI ``sage_flash_run``, include/sage_attn_run.h): S = Q K^T in
+fp32 from fp16/bf16 MFMAs, an online softmax, P rounded to V's dtype as the
+reference does (:87-88), P.V accumulated in fp32.  V rows 2^25 elements apart
+or more go through ``sage_vtiles`` and ``sage_flash_fwd`` instead.
 
 The library loader, argument checks and ``vtiles`` are the sage_attn pack's
 (loaded from the sibling pack by file path; packs have no parent package).
@@ -48,8 +48,12 @@ def run(q, k, v, causal=False, sm_scale=None, *, tensor_layout="HND", **kw):
     if sm_scale is None:
         sm_scale = D ** -0.5  # triton_impl.py:104-105
     qk_mul = float(np.float32(sm_scale * _H.LOG2E_REF))
-    vt = _H.vtiles(v, _PV_OF[q.dtype], tensor_layout=tensor_layout)
     o = _H._empty_like_layout(q, q.dtype)
+    if v.stride(2 if tensor_layout == "HND" else 1) < 1 << 25:
+        call = _H.pack_call(q, k, v, o, tensor_layout, (B, Hq, Hkv, Nq, Nkv, D), qk_mul, causal)
+        _H._check(lib.sage_flash_run(call, _H._stream(q.device)), "sage_flash_run")
+        return o
+    vt = _H.vtiles(v, _PV_OF[q.dtype], tensor_layout=tensor_layout)
     rc = lib.sage_flash_fwd(
         _H._ptr(q), _H._strides(q, tensor_layout), _H._ptr(k), _H._strides(k, tensor_layout),
         _H._ptr(vt), _H.DTYPE_VTILES, None, _H._ptr(o), _H._strides(o, tensor_layout),

@@ -24,6 +24,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import os
+import struct
 from pathlib import Path
 
 import numpy as np
@@ -110,6 +111,8 @@ def _load():
     lib.sage_flash_fwd.restype = i32
     lib.sage_flash_fwd.argtypes = [vp, p64, vp, p64, vp, i32, p64, vp, p64, i32, i64, i64, i64, i64, i64, i64, f32,
                                    i32, vp]
+    lib.sage_flash_run.restype = i32
+    lib.sage_flash_run.argtypes = [ctypes.c_char_p, vp]
     _LIB = lib
     return lib
 
@@ -146,6 +149,18 @@ def _ptr(t):
 
 def _stream(device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+_CALL = struct.Struct("@q4P18qd2q")  # sage_call (include/sage_attn_run.h)
+
+
+def pack_call(q, k, v, o, layout, dims, mul, causal) -> bytes:
+    """The sage_call of one whole call; dims = (B, Hq, Hkv, Nq, Nkv, D)."""
+    h, n = (1, 2) if layout == "HND" else (2, 1)
+    sq, sk, sv, so = q.stride(), k.stride(), v.stride(), o.stride()
+    return _CALL.pack(_CALL.size, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), sq[0], sq[h], sq[n],
+                      sk[0], sk[h], sk[n], sv[0], sv[h], sv[n], so[0], so[h], so[n], *dims, mul,
+                      _TORCH_CODES[q.dtype], int(bool(causal)))
 
 
 def _on_tensor_device(fn):
