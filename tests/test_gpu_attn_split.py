@@ -1,0 +1,93 @@
+"""Attention split over the keys (partial kernels and merge) against one sweep.
+
+``run`` chooses the split and the packing of grouped heads by the shape; the
+stage entry points (``attention`` on the pre-pass's own outputs, sage_flash_fwd
+on V tiles) always sweep all keys at once.  Q8, K8 and the scales are the same;
+P is rounded to its type against another running max (e_p = 2^-11 fp16, 2^-9
+bf16, 2^-4 e4m3, relative), the row sums of fp16 P carry 5 * 2^-11 each, and O
+is rounded to its type (e_o), so
+  |a - b| <= 2 e_p max|v| + (2 e_o + 10 * 2^-11) |o|.
+Shapes: single rows, rows that fill a tile with packed heads and ones that end
+in the middle of a head, keys that leave the last range short, causal rows that
+see nothing of a range, every Q-scale granularity, both layouts.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_gpu_flash_vrow import _flash, _tiles
+
+pytestmark = pytest.mark.gpu
+E = {"fp16": 2.0 ** -11, "bf16": 2.0 ** -9, "fp8": 2.0 ** -4}
+DT = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
+EO = {"bf16": 2.0 ** -9, "fp16": 2.0 ** -11, "fp32": 2.0 ** -24}
+
+# (B, Hq, Hkv, Nq, Nkv, causal)
+SHAPES = [(1, 1, 1, 1, 65, False), (1, 4, 1, 1, 4097, False), (2, 6, 2, 37, 3000, False),
+          (3, 8, 2, 32, 1000, False), (1, 12, 3, 127, 2111, False), (1, 2, 2, 130, 5000, False),
+          (1, 2, 1, 1500, 1500, True), (1, 3, 3, 777, 777, True)]
+
+
+def _inputs(shape, D, dtype, dev, seed=3):
+    B, Hq, Hkv, Nq, Nkv, _ = shape
+    g = torch.Generator().manual_seed(seed)
+    q = torch.randn(B, Hq, Nq, D, generator=g)
+    k = torch.randn(B, Hkv, Nkv, D, generator=g) + 2.0 * torch.randn(B, Hkv, 1, D, generator=g)
+    v = torch.randn(B, Hkv, Nkv, D, generator=g)
+    return [t.to(DT[dtype]).to(dev) for t in (q, k, v)]
+
+
+def _close(got, want, v, ep, eo):
+    torch.cuda.synchronize()
+    got, want = got.double(), want.double()
+    assert torch.isfinite(got).all()
+    bound = 2 * ep * v.double().abs().max() + (2 * eo + 10 * 2.0 ** -11) * want.abs()
+    worst = ((got - want).abs() / bound).max().item()
+    print(f"  worst error/bound {worst:.3f}")
+    assert worst <= 1.0
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(str(int(x)) for x in s))
+def test_int8_split_matches_one_sweep(shape, D, hip_impl, gpu_device):
+    causal = shape[5]
+    for i, (pv, gran, dtype) in enumerate([("fp16", "block", "bf16"), ("bf16", "wave", "fp16"),
+                                           ("fp8", "thread", "fp32")]):
+        print(f"[split] {shape} D{D} {pv} {gran} {dtype}", flush=True)
+        q, k, v = _inputs(shape, D, dtype, gpu_device)
+        layout = "NHD" if i == 1 else "HND"
+        if layout == "NHD":
+            q, k, v = (t.transpose(1, 2).contiguous() for t in (q, k, v))
+        o, pre = hip_impl.run(q, k, v, causal=causal, pv_dtype=pv, q_gran=gran, tensor_layout=layout, fuse_q=False,
+                              return_intermediates=True)
+        q_sub = hip_impl.q_sub_of(gran)
+        stage = hip_impl.prepass(q, k, v, q_sub=q_sub, pv_dtype=pv, tensor_layout=layout)
+        for key in ("q8", "q_scale", "k8", "k_scale", "km"):
+            assert torch.equal(pre[key], stage[key]), key
+        want = hip_impl.attention(q, k, v, stage, causal, pv_dtype=pv, q_sub=q_sub, tensor_layout=layout)
+        _close(o, want, v, E[pv], EO[dtype])
+        fused = hip_impl.run(q, k, v, causal=causal, pv_dtype=pv, q_gran=gran, tensor_layout=layout, fuse_q=True)
+        assert torch.equal(fused, o)  # where Q is quantized changes no bit
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(str(int(x)) for x in s))
+def test_flash_split_matches_one_sweep(shape, dtype, D, gpu_device):
+    print(f"[flash split] {shape} D{D} {dtype}", flush=True)
+    F = _flash()
+    q, k, v = _inputs(shape, D, dtype, gpu_device)
+    _close(F.run(q, k, v, causal=shape[5]), _tiles(F._H, q, k, v, shape[5]), v, E[dtype], EO[dtype])
+
+
+def test_split_handles_extreme_scores(gpu_device):
+    """A range whose scores are all far below another's weighs nothing; NaN
+    keys reach every row, as in one sweep."""
+    F = _flash()
+    q, k, v = _inputs((1, 1, 1, 3, 4096, False), 64, "fp16", gpu_device)
+    k[:, :, :2048] = 0
+    k[:, :, 2048:] = 200.0 * q[:, :, :1]
+    _close(F.run(q, k, v), _tiles(F._H, q, k, v, False), v, E["fp16"], EO["fp16"])
+    k[:, :, 4000] = float("nan")
+    assert torch.isnan(F.run(q, k, v)).all()

@@ -47,7 +47,8 @@ UNIT_FLAGS = {
     # LLVM's max-ilp machine-scheduler strategy for the attention kernels:
     # measured faster than the default at every configuration (A/B, one box:
     # config 2 +1.0 %, config 3 +1.2 %, config 4 +0.3 %, config 5 +2.2 %)
-    "sage_attn_fwd.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
+    **{f"sage_attn_{u}.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"] for u in ("i8", "i8q", "flash", "part")},
+    "sage_attn_fwd.hip": [],
     "sage_abi.hip": [],
     "sage_vtiles.hip": ["-ffp-contract=off"],
 }

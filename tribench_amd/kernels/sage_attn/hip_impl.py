@@ -111,8 +111,11 @@ def _load():
     lib.sage_flash_fwd.restype = i32
     lib.sage_flash_fwd.argtypes = [vp, p64, vp, p64, vp, i32, p64, vp, p64, i32, i64, i64, i64, i64, i64, i64, f32,
                                    i32, vp]
-    lib.sage_flash_run.restype = i32
-    lib.sage_flash_run.argtypes = [ctypes.c_char_p, vp]
+    for name in ("sage_run", "sage_flash_run"):
+        getattr(lib, name).restype = i32
+        getattr(lib, name).argtypes = [ctypes.c_char_p, vp]
+        getattr(lib, name + "_workspace_bytes").restype = sz
+        getattr(lib, name + "_workspace_bytes").argtypes = [ctypes.c_char_p]
     _LIB = lib
     return lib
 
@@ -151,16 +154,35 @@ def _stream(device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
-_CALL = struct.Struct("@q4P18qd2q")  # sage_call (include/sage_attn_run.h)
+_CALL = struct.Struct("@q6P18q1d6q6P6q")  # sage_call (include/sage_attn_run.h)
+_CALL_WS = struct.Struct("@2q")
+_CALL_WS_AT = 40  # byte offset of its workspace fields
 
 
-def pack_call(q, k, v, o, layout, dims, mul, causal) -> bytes:
-    """The sage_call of one whole call; dims = (B, Hq, Hkv, Nq, Nkv, D)."""
+def whole_call(fn, what, q, k, v, o, layout, dims, mul, causal, pv_mode=0, q_sub=0, smooth_k=0, fuse_q=0, outs=None):
+    """Run sage_run / sage_flash_run: pack the sage_call, allocate the
+    workspace it asks for and launch on the current stream.  dims = (B, Hq,
+    Hkv, Nq, Nkv, D); outs: q8, q_scale, k8, k_scale, km, v_scale tensors."""
+    lib = _load()
     h, n = (1, 2) if layout == "HND" else (2, 1)
     sq, sk, sv, so = q.stride(), k.stride(), v.stride(), o.stride()
-    return _CALL.pack(_CALL.size, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), sq[0], sq[h], sq[n],
-                      sk[0], sk[h], sk[n], sv[0], sv[h], sv[n], so[0], so[h], so[n], *dims, mul,
-                      _TORCH_CODES[q.dtype], int(bool(causal)))
+    if outs:
+        ptrs = [t.data_ptr() if t is not None else 0 for t in outs]
+        ptrs += [t.stride(i) if t is not None else 0 for t in (outs[0], outs[2]) for i in (0, h, n)]
+    else:
+        ptrs = _NO_OUTS
+    call = bytearray(_CALL.pack(
+        _CALL.size, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), 0, 0, sq[0], sq[h], sq[n], sk[0], sk[h],
+        sk[n], sv[0], sv[h], sv[n], so[0], so[h], so[n], *dims, mul, _TORCH_CODES[q.dtype], int(bool(causal)),
+        pv_mode, q_sub, smooth_k, fuse_q, *ptrs))
+    nbytes = getattr(lib, what + "_workspace_bytes")(bytes(call))
+    if nbytes:
+        ws = torch.empty((nbytes,), dtype=torch.uint8, device=q.device)
+        _CALL_WS.pack_into(call, _CALL_WS_AT, ws.data_ptr(), nbytes)
+    _check(fn(bytes(call), _stream(q.device)), what)
+
+
+_NO_OUTS = (0,) * 12
 
 
 def _on_tensor_device(fn):
@@ -446,26 +468,24 @@ def run(q, k, v, causal=False, sm_scale=None, *, pv_dtype="fp16", q_gran="block"
     if pv_dtype not in PV_MODES:
         raise ValueError(f"sage_attn hip: invalid argument: pv_dtype {pv_dtype!r}")
     q_sub = q_sub_of(q_gran)
-    _check_inputs(q, k, v, tensor_layout)
-    blkq, blkk = 128, 64  # BLOCK_M / BLOCK_N of triton_impl.py:166-167
-    if fuse_q is None:
-        fuse_q = fuse_q_default(_dims(q, tensor_layout)[3])
-    pre = prepass(q, k, v, sm_scale, blkq=blkq, blkk=blkk, q_sub=q_sub, smooth_k=smooth_k,
-                  pv_dtype=pv_dtype, quant_q=not fuse_q, tensor_layout=tensor_layout)
-    if fuse_q:
-        q8 = qs = None
-        if return_intermediates:
-            B, Hq, Nq, _ = _dims(q, tensor_layout)
-            q8 = _empty_like_layout(q, torch.int8)
-            qs = torch.empty((B, Hq, -(-Nq // blkq) * (blkq // q_sub)), dtype=torch.float32, device=q.device)
-            pre["q8"], pre["q_scale"] = q8, qs
-        o = attention_q(q, k, v, pre, causal, sm_scale, pv_dtype=pv_dtype, q_sub=q_sub, blkk=blkk,
-                        tensor_layout=tensor_layout, q8_out=q8, q_scale_out=qs)
-    else:
-        o = attention(q, k, v, pre, causal, pv_dtype=pv_dtype, q_sub=q_sub, blkq=blkq, blkk=blkk,
-                      tensor_layout=tensor_layout)
+    dims = _check_inputs(q, k, v, tensor_layout)
+    B, Hq, Hkv, Nq, Nkv, D = dims
+    lib = _load()
+    mul = float(np.float32((D ** -0.5 if sm_scale is None else sm_scale) * LOG2E_REF))
+    o = _empty_like_layout(q, q.dtype)
+    outs = None
     if return_intermediates:
-        for key in ("workspace", "vt", "vt_pv"):
-            pre.pop(key, None)
-        return o, pre
-    return o
+        pre = {"q8": _empty_like_layout(q, torch.int8),
+               "q_scale": torch.empty((B, Hq, -(-Nq // 128) * (128 // q_sub)), dtype=torch.float32, device=q.device),
+               "k8": _empty_like_layout(k, torch.int8),
+               "k_scale": torch.empty((B, Hkv, -(-Nkv // 64)), dtype=torch.float32, device=q.device)}
+        for key, on in (("km", smooth_k), ("v_scale", pv_dtype == "fp8")):
+            if on:
+                pre[key] = torch.empty((B, Hkv, D), dtype=torch.float32, device=q.device)
+        fuse_q = fuse_q_default(D) if fuse_q is None else fuse_q  # (where Q8 is written: see its strides)
+        if fuse_q and pre["q8"].stride() != q.stride():
+            raise ValueError("sage_attn hip: invalid argument: q8_out must be int8 with q's strides")
+        outs = [pre.get(key) for key in ("q8", "q_scale", "k8", "k_scale", "km", "v_scale")]
+    whole_call(lib.sage_run, "sage_run", q, k, v, o, tensor_layout, dims, mul, causal, PV_MODES[pv_dtype], q_sub,
+               int(bool(smooth_k)), -1 if fuse_q is None else int(bool(fuse_q)), outs)
+    return (o, pre) if return_intermediates else o
