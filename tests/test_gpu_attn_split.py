@@ -53,10 +53,15 @@ def _close(got, want, v, ep, eo):
 def test_int8_split_matches_one_sweep(shape, D, hip_impl, gpu_device):
     causal = shape[5]
     for i, (pv, gran, dtype) in enumerate([("fp16", "block", "bf16"), ("bf16", "wave", "fp16"),
-                                           ("fp8", "thread", "fp32")]):
+                                           ("fp8", "thread", "fp32"), ("fp16", "wave", "fp16"),
+                                           ("bf16", "thread", "bf16")]):  # the last two: V in place
         print(f"[split] {shape} D{D} {pv} {gran} {dtype}", flush=True)
         q, k, v = _inputs(shape, D, dtype, gpu_device)
-        layout = "NHD" if i == 1 else "HND"
+        layout = "NHD" if i in (1, 4) else "HND"
+        if i == 3:  # V rows that are slices of wider ones
+            wide = torch.zeros(*v.shape[:3], D + 24, dtype=v.dtype, device=v.device)
+            wide[..., :D] = v
+            v = wide[..., :D]
         if layout == "NHD":
             q, k, v = (t.transpose(1, 2).contiguous() for t in (q, k, v))
         o, pre = hip_impl.run(q, k, v, causal=causal, pv_dtype=pv, q_gran=gran, tensor_layout=layout, fuse_q=False,
@@ -79,6 +84,26 @@ def test_flash_split_matches_one_sweep(shape, dtype, D, gpu_device):
     F = _flash()
     q, k, v = _inputs(shape, D, dtype, gpu_device)
     _close(F.run(q, k, v, causal=shape[5]), _tiles(F._H, q, k, v, shape[5]), v, E[dtype], EO[dtype])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("N,causal", [(1, False), (64, False), (193, True), (577, False)])
+def test_int8_v_in_place_equals_tiles(N, causal, dtype, D, hip_impl, gpu_device):
+    """Enough heads for one sweep per work-group: V in place and V tiles then
+    do the same arithmetic, so the outputs are equal bit for bit."""
+    print(f"[int8 vrow] N{N} D{D} {dtype} causal={causal}", flush=True)
+    q, k, v = _inputs((16, 48, 48, N, N, causal), D, dtype, gpu_device)
+    o = hip_impl.run(q, k, v, causal=causal, pv_dtype=dtype)
+    stage = hip_impl.prepass(q, k, v, pv_dtype=dtype)
+    assert torch.equal(o, hip_impl.attention(q, k, v, stage, causal, pv_dtype=dtype))
+
+
+def test_int8_far_apart_v_rows_take_the_tile_path(hip_impl, gpu_device):
+    base = torch.randn((1 << 25) + 64, device=gpu_device, dtype=torch.float16)
+    v = base.as_strided((1, 1, 2, 64), (0, 0, 1 << 25, 1))
+    q, k = (torch.randn(1, 1, 2, 64, device=gpu_device, dtype=torch.float16) for _ in range(2))
+    assert torch.equal(hip_impl.run(q, k, v), hip_impl.run(q, k, v.contiguous()))
 
 
 def test_split_handles_extreme_scores(gpu_device):

@@ -284,6 +284,18 @@ extern "C" int sage_flash_fwd(const void* q, const int64_t* q_strides, const voi
   return launch_attn_flash(a, (int)D, in_dtype, 8, st, who);
 }
 
+// V read in place (sage_attn_kernel.h, kVRow)
+static bool vrow_ok(const sage_call& c) {
+  return c.v && (uintptr_t)c.v % 16 == 0 && strides_ok(c.v_strides, 2) && c.v_strides[2] < (1 << 25);
+}
+static void set_vrow(AttnArgs& a, const sage_call& c) {
+  a.v = c.v;
+  a.sv[0] = c.v_strides[0];
+  a.sv[1] = c.v_strides[1];
+  a.svn = (int)c.v_strides[2];
+  a.vrow = 1;
+}
+
 static bool call_ok(const sage_call* c) { return c && c->size == (int64_t)sizeof(sage_call); }
 static bool shape_ok(const sage_call* c) {
   return c->B > 0 && c->Hq > 0 && c->Hkv > 0 && c->Nq > 0 && c->Nkv > 0 && c->Hq % c->Hkv == 0;
@@ -301,13 +313,9 @@ extern "C" int sage_flash_run(const sage_call* c, void* stream) {
   if (int rc = flash_setup(a, who, c->q, c->q_strides, c->k, c->k_strides, c->o, c->o_strides, (int)c->dtype, c->B,
                            c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, (float)c->mul, (int)c->causal))
     return rc;
-  if (!c->v || (uintptr_t)c->v % 16 != 0 || !strides_ok(c->v_strides, 2) || c->v_strides[2] >= (1 << 25))
+  if (!vrow_ok(*c))
     return fail("%s: invalid argument: V must have 16-byte aligned rows less than 2^25 elements apart", who);
-  a.v = c->v;
-  a.sv[0] = c->v_strides[0];
-  a.sv[1] = c->v_strides[1];
-  a.svn = (int)c->v_strides[2];
-  a.vrow = 1;
+  set_vrow(a, *c);
   const AttnPlan p = attn_plan(c->B, c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, c->causal != 0, false, 0, true);
   const size_t need = part_bytes(p, c->B, c->Hq, c->Nq, c->D);
   if (need && (!c->workspace || (size_t)c->workspace_bytes < need || (uintptr_t)c->workspace % 256 != 0))
@@ -328,15 +336,16 @@ namespace sage {
 // AttnArgs of a sage_run call: INT8 Q from the pre-pass (quantized) or Q itself.
 static int attn_args(AttnArgs& a, const char* who, const sage_call& c, bool quantized, int8_t* q8,
                      const int64_t* q8_strides, float* qs, const int8_t* k8, const int64_t* k8_strides,
-                     const float* ks, const void* vt, const float* vs) {
+                     const float* ks, const void* vt, const float* vs) {  // vt NULL: V read in place
   const float mul = (float)c.mul;
   const int qes = quantized ? 1 : (c.dtype == SAGE_DTYPE_F32 ? 4 : 2);
-  if (int rc = attn_setup(a, who, quantized ? q8_strides : c.q_strides, qes, k8, k8_strides, ks, vt,
+  if (int rc = attn_setup(a, who, quantized ? q8_strides : c.q_strides, qes, k8, k8_strides, ks, vt ? vt : c.v,
                           SAGE_DTYPE_VTILES, vs, c.o, (int)c.dtype, c.o_strides, c.B, c.Hq, c.Hkv, c.Nq, c.Nkv, c.D,
                           (int)c.causal, 128, 64, (int)c.q_sub, (int)c.pv_mode))
     return rc;
   if (((uintptr_t)c.q | (uintptr_t)q8) % 16 != 0)
     return fail("%s: invalid argument: base pointers must be 16-byte aligned", who);
+  if (!vt) set_vrow(a, c);
   if (quantized) {
     a.q8 = q8;
     a.q_scale = qs;
@@ -355,6 +364,7 @@ struct RunPlan {
   AttnPlan attn;
   bool fuse_q;   // Q quantized in the prologue, if the attention's plan allows it
   bool quant_q;  // Q quantized in the pre-pass
+  bool vrow;     // V read in place instead of through V tiles
   int v_mode;
   size_t off_q8, off_qs, off_k8, off_ks, off_km, off_vs, off_pre, off_vt, off_part, pre_bytes, vt_bytes, bytes;
 };
@@ -369,9 +379,16 @@ static RunPlan run_plan(const sage_call* c) {
   // N159 D128: 24.6 us against 26.8).
   r.fuse_q = c->fuse_q < 0 ? (c->Nq + 127) / 128 * c->Hq * c->B > 256 : c->fuse_q != 0;
   r.quant_q = !r.fuse_q || r.attn.part();  // the partial kernels read Q8
+  // V already in the P.V type: read in place, no V tiles (4 bytes of traffic
+  // per element less: fp16 B8 H16 N4096 D64 548 us -> 536, 32 rows over 16384
+  // keys B2 8 KV heads D128 99 -> 87, B1 H24 N1333 D128 51.7 -> 49.8; no shape
+  // measured slower by more than its runs differ)
+  r.vrow = ((c->dtype == SAGE_DTYPE_F16 && c->pv_mode == SAGE_PV_F16) ||
+            (c->dtype == SAGE_DTYPE_BF16 && c->pv_mode == SAGE_PV_BF16)) &&
+           vrow_ok(*c);
   r.v_mode = c->pv_mode == SAGE_PV_FP8 ? SAGE_V_FP8_SCALE : SAGE_V_NONE;
   r.pre_bytes = sage_prepass_workspace_bytes(c->B, c->Hkv, c->Nkv, c->D, (int)c->smooth_k, r.v_mode);
-  r.vt_bytes = sage_vtile_bytes(c->B, c->Hkv, c->Nkv, c->D, (int)c->pv_mode);
+  r.vt_bytes = r.vrow ? 0 : sage_vtile_bytes(c->B, c->Hkv, c->Nkv, c->D, (int)c->pv_mode);
   size_t at = 0;
   auto take = [&](size_t n) {
     const size_t o = at;
@@ -429,14 +446,14 @@ extern "C" int sage_run(const sage_call* c, void* stream) {
   const float mul = (float)c->mul;
   if (r.fuse_q && (!(mul > 0.0f) || mul == INFINITY)) return fail("%s: invalid argument: mul %g", who, mul);
 
-  const void* vt = ws + r.off_vt;
   const int pv = (int)c->pv_mode, dt = (int)c->dtype, q_sub = (int)c->q_sub;
   const bool dq = r.quant_q;
-  if (int rc = sage_prepass_vt(dq ? c->q : nullptr, c->k, c->v, dt, c->B, c->Hq, c->Hkv, c->Nq, c->Nkv, c->D,
-                               dq ? c->q_strides : nullptr, c->k_strides, c->v_strides, mul, 128, 64, q_sub,
-                               (int)c->smooth_k, r.v_mode, dq ? q8 : nullptr, dq ? q8_strides : nullptr,
-                               dq ? qs : nullptr, k8, k8_strides, ks, km, nullptr, nullptr, vs, ws + r.off_pre,
-                               r.pre_bytes, pv, ws + r.off_vt, r.vt_bytes, stream))
+  void* vt = r.vrow ? nullptr : ws + r.off_vt;
+  if (int rc = prepass_any(who, dq ? c->q : nullptr, c->k, r.vrow ? nullptr : c->v, dt, c->B, c->Hq, c->Hkv, c->Nq,
+                           c->Nkv, c->D, dq ? c->q_strides : nullptr, c->k_strides, c->v_strides, mul, 128, 64, q_sub,
+                           (int)c->smooth_k, r.v_mode, dq ? q8 : nullptr, dq ? q8_strides : nullptr,
+                           dq ? qs : nullptr, k8, k8_strides, ks, km, nullptr, nullptr, vs, ws + r.off_pre,
+                           r.pre_bytes, pv, vt, r.vt_bytes, stream))
     return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   AttnArgs a{};

@@ -343,7 +343,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   // the kernel being measured; a global store would enter the vmcnt
   // accounting of the tile loads) and to the trace buffer at the end.  A
   // kernel whose tile ring leaves no room for them is not traced.
-  constexpr bool kTrace = RING + SINK + QAMAX + NW * kTraceWords * 8 <= 160 * 1024;
+  constexpr bool kTrace = NW == 8 && !kPart && RING + SINK + QAMAX + NW * kTraceWords * 8 <= 160 * 1024;
   unsigned long long* tr_s = nullptr;
   if constexpr (kTrace) tr_s = trace_lds<NW>();
   // every lane stores the same wave-uniform value (no branch around the store)
@@ -1198,17 +1198,21 @@ int launch_attn_nw(const AttnArgs& a, hipStream_t st, const char* who) {
   return check_launch(who);
 }
 
-// every (head dim, P.V type, output type) of one INT8 kernel
+// every (head dim, P.V type, output type) of one INT8 kernel; V in place
+// when the input (and output) type is the P.V type
+template <int QKM, int D, typename TO, int NW>
+int launch_attn_int8_d(const AttnArgs& a, int pv_mode, hipStream_t st, const char* who) {
+  constexpr int kRowPv = std::is_same_v<TO, _Float16> ? SAGE_PV_F16 : SAGE_PV_BF16;
+  if constexpr (!std::is_same_v<TO, float>)
+    if (a.vrow) return launch_attn_nw<QKM, D, kRowPv, TO, NW, true>(a, st, who);
+  if (pv_mode == SAGE_PV_F16) return launch_attn_nw<QKM, D, SAGE_PV_F16, TO, NW, false>(a, st, who);
+  if (pv_mode == SAGE_PV_BF16) return launch_attn_nw<QKM, D, SAGE_PV_BF16, TO, NW, false>(a, st, who);
+  return launch_attn_nw<QKM, D, SAGE_PV_FP8, TO, NW, false>(a, st, who);
+}
 template <int QKM, typename TO, int NW>
 int launch_attn_int8(const AttnArgs& a, int D, int pv_mode, hipStream_t st, const char* who) {
-  if (D == 64) {
-    if (pv_mode == SAGE_PV_F16) return launch_attn_nw<QKM, 64, SAGE_PV_F16, TO, NW, false>(a, st, who);
-    if (pv_mode == SAGE_PV_BF16) return launch_attn_nw<QKM, 64, SAGE_PV_BF16, TO, NW, false>(a, st, who);
-    return launch_attn_nw<QKM, 64, SAGE_PV_FP8, TO, NW, false>(a, st, who);
-  }
-  if (pv_mode == SAGE_PV_F16) return launch_attn_nw<QKM, 128, SAGE_PV_F16, TO, NW, false>(a, st, who);
-  if (pv_mode == SAGE_PV_BF16) return launch_attn_nw<QKM, 128, SAGE_PV_BF16, TO, NW, false>(a, st, who);
-  return launch_attn_nw<QKM, 128, SAGE_PV_FP8, TO, NW, false>(a, st, who);
+  return D == 64 ? launch_attn_int8_d<QKM, 64, TO, NW>(a, pv_mode, st, who)
+                 : launch_attn_int8_d<QKM, 128, TO, NW>(a, pv_mode, st, who);
 }
 template <int QKM, typename TO>
 int launch_attn_int8(const AttnArgs& a, int D, int pv_mode, int nw, hipStream_t st, const char* who) {

@@ -75,7 +75,10 @@ template <int D>
 static int launch_part_d(const AttnArgs& a, int pv_mode, bool i8, int o_dtype, hipStream_t st, const char* who) {
   int rc;
   if (i8) {
-    if (pv_mode == SAGE_PV_F16) rc = launch_part<kQkI8, D, SAGE_PV_F16, false>(a, st, who);
+    if (a.vrow)
+      rc = pv_mode == SAGE_PV_F16 ? launch_part<kQkI8, D, SAGE_PV_F16, true>(a, st, who)
+                                  : launch_part<kQkI8, D, SAGE_PV_BF16, true>(a, st, who);
+    else if (pv_mode == SAGE_PV_F16) rc = launch_part<kQkI8, D, SAGE_PV_F16, false>(a, st, who);
     else if (pv_mode == SAGE_PV_BF16) rc = launch_part<kQkI8, D, SAGE_PV_BF16, false>(a, st, who);
     else rc = launch_part<kQkI8, D, SAGE_PV_FP8, false>(a, st, who);
   } else if (o_dtype == SAGE_DTYPE_F16) {

@@ -133,4 +133,12 @@ __device__ __forceinline__ uint32_t group_max_u32(uint32_t v) {
 namespace sage {
 int fail(const char* fmt, ...);
 int check_launch(const char* what);
+
+// sage_prepass (vt NULL) or sage_prepass_vt, reporting errors as `who`
+int prepass_any(const char* who, const void* q, const void* k, const void* v, int in_dtype, int64_t B, int64_t Hq,
+                int64_t Hkv, int64_t Nq, int64_t Nkv, int64_t D, const int64_t* q_strides, const int64_t* k_strides,
+                const int64_t* v_strides, float q_mul, int blkq, int blkk, int q_sub, int smooth_k, int v_mode,
+                int8_t* q8, const int64_t* q8_strides, float* q_scale, int8_t* k8, const int64_t* k8_strides,
+                float* k_scale, float* km, uint8_t* v8, const int64_t* v8_strides, float* v_scale, void* workspace,
+                size_t workspace_bytes, int pv_mode, void* vt, size_t vt_bytes, void* stream);
 }  // namespace sage

@@ -558,7 +558,7 @@ extern "C" size_t sage_prepass_workspace_bytes(int64_t B, int64_t Hkv, int64_t N
   return bytes;
 }
 
-static int prepass_impl(const char* who, const void* q, const void* k, const void* v, int in_dtype, int64_t B,
+int sage::prepass_any(const char* who, const void* q, const void* k, const void* v, int in_dtype, int64_t B,
                         int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nkv, int64_t D, const int64_t* q_strides,
                         const int64_t* k_strides, const int64_t* v_strides, float q_mul, int blkq, int blkk,
                         int q_sub, int smooth_k, int v_mode, int8_t* q8, const int64_t* q8_strides, float* q_scale,
@@ -692,7 +692,7 @@ extern "C" int sage_prepass(const void* q, const void* k, const void* v, int in_
                             float* q_scale, int8_t* k8, const int64_t* k8_strides, float* k_scale,
                             float* km, uint8_t* v8, const int64_t* v8_strides, float* v_scale,
                             void* workspace, size_t workspace_bytes, void* stream) {
-  return prepass_impl("sage_prepass", q, k, v, in_dtype, B, Hq, Hkv, Nq, Nkv, D, q_strides, k_strides, v_strides,
+  return prepass_any("sage_prepass", q, k, v, in_dtype, B, Hq, Hkv, Nq, Nkv, D, q_strides, k_strides, v_strides,
                       q_mul, blkq, blkk, q_sub, smooth_k, v_mode, q8, q8_strides, q_scale, k8, k8_strides, k_scale,
                       km, v8, v8_strides, v_scale, workspace, workspace_bytes, -1, nullptr, 0, stream);
 }
@@ -707,7 +707,7 @@ extern "C" int sage_prepass_vt(const void* q, const void* k, const void* v, int 
                                void* workspace, size_t workspace_bytes, int pv_mode, void* vtiles,
                                size_t vtile_bytes, void* stream) {
   if (!vtiles) return fail("sage_prepass_vt: invalid argument: null pointer (vtiles)");
-  return prepass_impl("sage_prepass_vt", q, k, v, in_dtype, B, Hq, Hkv, Nq, Nkv, D, q_strides, k_strides,
+  return prepass_any("sage_prepass_vt", q, k, v, in_dtype, B, Hq, Hkv, Nq, Nkv, D, q_strides, k_strides,
                       v_strides, q_mul, blkq, blkk, q_sub, smooth_k, v_mode, q8, q8_strides, q_scale, k8,
                       k8_strides, k_scale, km, v8, v8_strides, v_scale, workspace, workspace_bytes, pv_mode, vtiles,
                       vtile_bytes, stream);
@@ -767,7 +767,7 @@ extern "C" int sage_prepass_vt_noalloc(const void* q, const void* k, const void*
                 who, need, (size_t)SAGE_SCRATCH_BYTES);
   void* ws = nullptr;
   if (int rc = scratch_address(who, &ws)) return rc;
-  return prepass_impl(who, q, k, v, in_dtype, B, Hq, Hkv, Nq, Nkv, D, q_strides, k_strides, v_strides, q_mul,
+  return prepass_any(who, q, k, v, in_dtype, B, Hq, Hkv, Nq, Nkv, D, q_strides, k_strides, v_strides, q_mul,
                       blkq, blkk, q_sub, smooth_k, v_mode, q8, q8_strides, q_scale, k8, k8_strides, k_scale, km, v8,
                       v8_strides, v_scale, ws, SAGE_SCRATCH_BYTES, pv_mode, vtiles, vtile_bytes, stream);
 }
