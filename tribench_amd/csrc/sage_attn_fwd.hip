@@ -17,7 +17,7 @@ int64_t g_trace_words = 0;
 // a work-group's rows, key ranges.
 // ---------------------------------------------------------------------------
 struct AttnPlan {
-  int nw = 8, grp = 1, nsplit = 1;
+  int nw = 8, wpe = 2, grp = 1, nsplit = 1;
   bool part() const { return grp > 1 || nsplit > 1; }
 };
 
@@ -35,7 +35,7 @@ struct AttnPlan {
 // against 332); splits and packed heads fill the chip when rows are few (one
 // row, 4 heads to a KV head, 8192 keys: 52 us against 146).
 static AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nkv, int64_t D, bool causal,
-                          bool i8, int pv_mode, bool may_split) {
+                          bool i8, int pv_mode, int dtype, bool may_split) {
   const double start8 = 5.5, start4 = 4.0, split_us = 3.6, merge_bytes_per_us = 7.4e6;
   double blk8 = 0.48, blk4 = 0.46;
   if (D == 128) {
@@ -46,7 +46,9 @@ static AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_
   // blocks of a work-group: all of them, or with causal rows over several rounds the mean
   auto sweep = [&](int64_t wgs, int64_t slots, double start, double blk, int64_t nsplit) {
     const double blocks = causal && wgs > slots ? 0.5 * (double)(nt + 2) : (double)nt;
-    return (double)((wgs + slots - 1) / slots) * (start + ceil(blocks / (double)nsplit) * blk);
+    // (over many rounds the work-groups' ends spread and the last round fills)
+    const double full = (double)wgs / (double)slots;
+    return (full < 3.0 ? ceil(full) : full) * (start + ceil(blocks / (double)nsplit) * blk);
   };
   AttnPlan best;
   double t = sweep((Nq + 255) / 256 * Hq * B, 256, start8, blk8, 1);
@@ -57,11 +59,25 @@ static AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_
     if (c < t) {
       t = c;
       best.nw = 4;
+      best.wpe = 2;
       best.grp = grp;
       best.nsplit = nsplit;
     }
   };
   consider(1, 1);
+  // (FP8 P with fp32 outputs spills there: 685 us -> 794 at B4 H48 N3801)
+  if (D == 64 && !(i8 && pv_mode == SAGE_PV_FP8 && dtype == SAGE_DTYPE_F32)) {
+    // Three 4-wave work-groups to a CU hide more of each one's start, without
+    // the second S buffer (168 VGPRs): a block takes 1.5x (INT8) to 1.7x as
+    // long, shared by three.  226 keys: 267 us -> 215 per call (B2 H48
+    // N17776), 697 keys 110 -> 99 (B3 H12 N10198); at 8070 keys 571 -> 620.
+    const double c = sweep((Nq + 127) / 128 * Hq * B, 768, start4, i8 ? 0.71 : 0.85, 1);
+    if (c < t) {
+      t = c;
+      best.nw = 4;
+      best.wpe = 3;
+    }
+  }
   if (!may_split) return best;
   for (const int nsplit : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32}) {
     if (nsplit > nt) break;
@@ -150,11 +166,13 @@ static int attn_setup(AttnArgs& a, const char* who, const int64_t* q_strides, in
 }
 
 // waves per work-group of the entry points that have no workspace
-static int stage_nw(const AttnArgs& a, int64_t D, int pv_mode) {
+static int stage_nw(AttnArgs& a, int64_t D, int pv_mode, int dtype) {
 #if SAGE_TRACE
   return 8;
 #endif
-  return attn_plan(a.B, a.Hq, a.Hkv, a.Nq, a.Nkv, D, a.causal != 0, true, pv_mode, false).nw;
+  const AttnPlan p = attn_plan(a.B, a.Hq, a.Hkv, a.Nq, a.Nkv, D, a.causal != 0, true, pv_mode, dtype, false);
+  a.wpe = p.wpe;
+  return p.nw;
 }
 
 }  // namespace sage
@@ -178,7 +196,7 @@ extern "C" int sage_attn_fwd(const int8_t* q8, const int64_t* q8_strides, const 
   a.q8 = q8;
   a.q_scale = q_scale;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return launch_attn_i8(a, (int)D, pv_mode, o_dtype, stage_nw(a, D, pv_mode), st, who);
+  return launch_attn_i8(a, (int)D, pv_mode, o_dtype, stage_nw(a, D, pv_mode, o_dtype), st, who);
 }
 
 extern "C" int sage_attn_fwd_q(const void* q, const int64_t* q_strides, int q_dtype, float q_mul, int8_t* q8_out,
@@ -205,7 +223,7 @@ extern "C" int sage_attn_fwd_q(const void* q, const int64_t* q_strides, int q_dt
   a.q8_out = q8_out;
   a.qs_out = q_scale_out;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return launch_attn_i8q(a, (int)D, pv_mode, q_dtype, stage_nw(a, D, pv_mode), st, who);
+  return launch_attn_i8q(a, (int)D, pv_mode, q_dtype, stage_nw(a, D, pv_mode, q_dtype), st, who);
 }
 
 #if SAGE_TRACE
@@ -303,7 +321,7 @@ static bool shape_ok(const sage_call* c) {
 
 extern "C" size_t sage_flash_run_workspace_bytes(const sage_call* c) {
   if (!call_ok(c) || !shape_ok(c)) return 0;
-  return part_bytes(attn_plan(c->B, c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, c->causal != 0, false, 0, true), c->B, c->Hq, c->Nq, c->D);
+  return part_bytes(attn_plan(c->B, c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, c->causal != 0, false, 0, (int)c->dtype, true), c->B, c->Hq, c->Nq, c->D);
 }
 
 extern "C" int sage_flash_run(const sage_call* c, void* stream) {
@@ -316,7 +334,7 @@ extern "C" int sage_flash_run(const sage_call* c, void* stream) {
   if (!vrow_ok(*c))
     return fail("%s: invalid argument: V must have 16-byte aligned rows less than 2^25 elements apart", who);
   set_vrow(a, *c);
-  const AttnPlan p = attn_plan(c->B, c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, c->causal != 0, false, 0, true);
+  const AttnPlan p = attn_plan(c->B, c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, c->causal != 0, false, 0, (int)c->dtype, true);
   const size_t need = part_bytes(p, c->B, c->Hq, c->Nq, c->D);
   if (need && (!c->workspace || (size_t)c->workspace_bytes < need || (uintptr_t)c->workspace % 256 != 0))
     return fail("%s: invalid argument: workspace (%zu bytes, 256-byte aligned)", who, need);
@@ -328,6 +346,7 @@ extern "C" int sage_flash_run(const sage_call* c, void* stream) {
     part_setup(a, p, c->D, static_cast<char*>(c->workspace));
     return launch_attn_part(a, (int)c->D, 0, false, (int)c->dtype, st, who);
   }
+  a.wpe = p.wpe;
   return launch_attn_flash(a, (int)c->D, (int)c->dtype, p.nw, st, who);
 }
 
@@ -371,7 +390,7 @@ struct RunPlan {
 
 static RunPlan run_plan(const sage_call* c) {
   RunPlan r;
-  r.attn = attn_plan(c->B, c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, c->causal != 0, true, (int)c->pv_mode, true);
+  r.attn = attn_plan(c->B, c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, c->causal != 0, true, (int)c->pv_mode, (int)c->dtype, true);
   // The prologue saves a pass over Q (written and read again) and lengthens
   // each work-group's start: with more 128-row blocks than CUs it is 1 to 18 %
   // faster per call (226 keys, B2 H48 N17776 D64: 267 us against 292), with
@@ -466,6 +485,7 @@ extern "C" int sage_run(const sage_call* c, void* stream) {
     part_setup(a, r.attn, c->D, ws + r.off_part);
     return launch_attn_part(a, (int)c->D, pv, true, dt, st, who);
   }
+  a.wpe = r.attn.wpe;
   return dq ? launch_attn_i8(a, (int)c->D, pv, dt, r.attn.nw, st, who)
             : launch_attn_i8q(a, (int)c->D, pv, dt, r.attn.nw, st, who);
 }

@@ -89,6 +89,7 @@ struct AttnArgs {
   // work-group's rows (row r is row r % Nq of head r / Nq of the group), the
   // keys are split into `nsplit` ranges
   int grp, nsplit;
+  int wpe;         // host only: waves per SIMD of a 4-wave launch at D = 64 (3, else 2)
   float* part_o;   // [nsplit][B*Hq*Nq][D] sum of p * v against the split's own max
   float2* part_ml; // [nsplit][B*Hq*Nq] that max (log2 units) and the sum of p
 #if SAGE_TRACE
@@ -290,11 +291,13 @@ __device__ __forceinline__ int vrow_swz(int r) {
 // alternating with the one ring: 925 -> 910 us at B4 H32 N4096 D128, 571 -> 563
 // at B8 H16 N4096 D64 (4-slot rings: a trip of the unrolled loop is 4
 // iterations, not 10), 1062 -> 1029 unquantized at B4 H32 N4096 D128.
-template <int QKM, int D, int PVM, int NW>
+// WPE (waves per SIMD) 3: three 4-wave work-groups to a CU, D = 64 only.
+template <int QKM, int D, int PVM, int NW, int WPE>
 struct TileRing {
   static constexpr bool kI8 = QKM == kQkI8 || QKM == kQkI8Q;
-  static constexpr int NK = D == 64 ? 4 : 3;
-  static constexpr int NV = D == 64 ? 4 : (kI8 ? 3 : 2);
+  static constexpr bool kFour = D == 64 && (kI8 || WPE == 2);  // (three work-groups to a CU: 53 KB each)
+  static constexpr int NK = kFour ? 4 : 3;
+  static constexpr int NV = kFour ? 4 : (kI8 || D == 64 ? 3 : 2);
   static constexpr int kVA = NV > 2 ? 1 : 0;
 };
 
@@ -302,8 +305,8 @@ struct TileRing {
 // each) of one (batch, head); Q rows, S, P and the O^T accumulators live in
 // arch VGPRs.  Tiles of 64 keys (K rows and V^T rows) reach LDS by direct
 // global -> LDS loads, two iterations ahead of their use (TileRing).
-template <int QKM, int D, int PVM, typename TO, int NW, bool kVRow, bool kPart>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_kernel(AttnArgs a) {
+template <int QKM, int D, int PVM, typename TO, int NW, int WPE, bool kVRow, bool kPart>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void attn_fwd_kernel(AttnArgs a) {
   constexpr int BM = 32 * NW;  // query rows per work-group
   constexpr bool kFQ = QKM == kQkI8Q;  // Q quantized in the prologue
   constexpr bool kI8 = QKM == kQkI8 || kFQ;
@@ -319,7 +322,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   constexpr int VRB = 64 * EB;      // V^T row bytes
   constexpr int KTB = kBN * KRB;    // K tile bytes
   constexpr int VTB = D * VRB;      // V^T tile bytes
-  using Ring = TileRing<QKM, D, PVM, NW>;
+  using Ring = TileRing<QKM, D, PVM, NW, WPE>;
   constexpr int NK = Ring::NK, NV = Ring::NV, kVA = Ring::kVA;
   constexpr int VOFF = NK * KTB;                  // V tiles follow the K tiles
   constexpr int RING = NK * KTB + NV * VTB;
@@ -931,7 +934,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     sync_tiles(true, true, true);
   };
 
-  // INT8 with fp16 P, and fp16/bf16 QK at D = 64: the S of block j+1 goes to
+  // With two waves per SIMD, INT8 with fp16 P and fp16/bf16 QK at D = 64: the S of block j+1 goes to
   // a second buffer, so that its QK MFMAs share one basic block with the P.V
   // MFMAs of block j-1 and the softmax of block j (the scheduler interleaves
   // all three; measured -1.9 % per launch at config 2, -1.2 % at config 4,
@@ -939,7 +942,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   // fp16/bf16 QK at D = 128 has no registers left for it).  Two iterations
   // per trip swap the buffers' roles (ten at D = 64, where the ring slots are
   // constants too).  sl as for fast_iter.
-  constexpr bool kTwoS = (kI8 && PVM == SAGE_PV_F16) || (!kI8 && D == 64);
+  constexpr bool kTwoS = WPE == 2 && ((kI8 && PVM == SAGE_PV_F16) || (!kI8 && D == 64));
   static_assert(!(kTwoS && PVM == SAGE_PV_FP8), "fused_iter uses the fp16/bf16 P shortcut of softmax_fast_on");
   SAcc S2[2];
   float ksc2 = 0.0f;
@@ -1070,13 +1073,21 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   int j = 1;
   // D = 64: constant ring slots, j % 4 == 1 at every trip (at D = 128 the
   // copies run out of registers); the two S buffers swap every iteration
-  static_assert(D != 64 || (NK == 4 && NV == 4), "unrolled by the ring");
+  static_assert(!(kTwoS && D == 64) || (NK == 4 && NV == 4), "unrolled by the ring");
+  static_assert(D != 64 || NK == NV, "one slot index");
   if constexpr (kTwoS && D == 64)
     for (; j + 4 <= j_fast; j += 4) {
       fused_iter(j, 1, S, ksc_cur, S2, ksc2);
       fused_iter(j + 1, 2, S2, ksc2, S, ksc_cur);
       fused_iter(j + 2, 3, S, ksc_cur, S2, ksc2);
       fused_iter(j + 3, 0, S2, ksc2, S, ksc_cur);
+    }
+  if constexpr (!kTwoS && D == 64 && PVM == SAGE_PV_F16)
+    for (; j + NK <= j_fast; j += NK) {
+      fast_iter(j, 1);
+      fast_iter(j + 1, 2);
+      fast_iter(j + 2, 3 % NK);
+      if constexpr (NK == 4) fast_iter(j + 3, 0);
     }
   if constexpr (kTwoS && D == 128)
     for (; j + 2 <= j_fast; j += 2) {
@@ -1178,8 +1189,8 @@ extern unsigned long long* g_trace;
 extern int64_t g_trace_words;
 #endif
 
-template <int QKM, int D, int PVM, typename TO, int NW, bool kVRow>
-int launch_attn_nw(const AttnArgs& a, hipStream_t st, const char* who) {
+template <int QKM, int D, int PVM, typename TO, int NW, int WPE, bool kVRow>
+int launch_attn_wpe(const AttnArgs& a, hipStream_t st, const char* who) {
   const int64_t nqb = (a.Nq + 32 * NW - 1) / (32 * NW);
   const int64_t grid = nqb * a.Hq * a.B;
   if (grid > 0x7FFFFFFF) return fail("%s: invalid argument: grid too large", who);
@@ -1189,13 +1200,20 @@ int launch_attn_nw(const AttnArgs& a, hipStream_t st, const char* who) {
   if (at.trace && grid * NW * kTraceWords > g_trace_words)
     return fail("%s: invalid argument: trace buffer of %lld words < %lld", who, (long long)g_trace_words,
                 (long long)(grid * NW * kTraceWords));
-  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW, kVRow, false>), dim3((unsigned)grid), dim3(64 * NW), 0, st,
+  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW, WPE, kVRow, false>), dim3((unsigned)grid), dim3(64 * NW), 0, st,
                      at);
 #else
-  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW, kVRow, false>), dim3((unsigned)grid), dim3(64 * NW), 0, st,
+  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, TO, NW, WPE, kVRow, false>), dim3((unsigned)grid), dim3(64 * NW), 0, st,
                      a);
 #endif
   return check_launch(who);
+}
+
+template <int QKM, int D, int PVM, typename TO, int NW, bool kVRow>
+int launch_attn_nw(const AttnArgs& a, hipStream_t st, const char* who) {
+  if constexpr (D == 64 && NW == 4)
+    if (a.wpe == 3) return launch_attn_wpe<QKM, D, PVM, TO, NW, 3, kVRow>(a, st, who);
+  return launch_attn_wpe<QKM, D, PVM, TO, NW, 2, kVRow>(a, st, who);
 }
 
 // every (head dim, P.V type, output type) of one INT8 kernel; V in place

@@ -17,7 +17,7 @@ static int launch_part(const AttnArgs& a, hipStream_t st, const char* who) {
   const int64_t rows = (int64_t)a.grp * a.Nq;
   const int64_t grid = (rows + 127) / 128 * (a.Hq / a.grp) * a.B * a.nsplit;
   if (grid > 0x7FFFFFFF) return fail("%s: invalid argument: grid too large", who);
-  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, float, 4, kVRow, true>), dim3((unsigned)grid), dim3(256), 0, st, a);
+  hipLaunchKernelGGL((attn_fwd_kernel<QKM, D, PVM, float, 4, 2, kVRow, true>), dim3((unsigned)grid), dim3(256), 0, st, a);
   return check_launch(who);
 }
 
