@@ -50,8 +50,8 @@ def run(q, k, v, causal=False, sm_scale=None, *, tensor_layout="HND", **kw):
     qk_mul = float(np.float32(sm_scale * _H.LOG2E_REF))
     o = _H._empty_like_layout(q, q.dtype)
     if v.stride(2 if tensor_layout == "HND" else 1) < 1 << 25:
-        _H.whole_call(lib.sage_flash_run, "sage_flash_run", q, k, v, o, tensor_layout, (B, Hq, Hkv, Nq, Nkv, D),
-                      qk_mul, causal)
+        _H.whole_call(lib.sage_flash_run, lib.sage_flash_run_workspace_bytes, "sage_flash_run", q, k, v, o,
+                      tensor_layout, (B, Hq, Hkv, Nq, Nkv, D), qk_mul, causal)
         return o
     vt = _H.vtiles(v, _PV_OF[q.dtype], tensor_layout=tensor_layout)
     rc = lib.sage_flash_fwd(

@@ -155,15 +155,18 @@ def _stream(device) -> ctypes.c_void_p:
 
 
 _CALL = struct.Struct("@q6P18q1d6q6P6q")  # sage_call (include/sage_attn_run.h)
+_CALL_SIZE = _CALL.size
 _CALL_WS = struct.Struct("@2q")
+_raw_stream = torch._C._cuda_getCurrentRawStream  # the handle alone: no Stream object per call
 _CALL_WS_AT = 40  # byte offset of its workspace fields
 
 
-def whole_call(fn, what, q, k, v, o, layout, dims, mul, causal, pv_mode=0, q_sub=0, smooth_k=0, fuse_q=0, outs=None):
+def whole_call(fn, fn_bytes, what, q, k, v, o, layout, dims, mul, causal, pv_mode=0, q_sub=0, smooth_k=0, fuse_q=0, outs=None):
     """Run sage_run / sage_flash_run: pack the sage_call, allocate the
     workspace it asks for and launch on the current stream.  dims = (B, Hq,
     Hkv, Nq, Nkv, D); outs: q8, q_scale, k8, k_scale, km, v_scale tensors."""
-    lib = _load()
+    if layout not in ("HND", "NHD"):
+        raise ValueError(f"sage_attn hip: invalid argument: tensor_layout {layout!r}")
     h, n = (1, 2) if layout == "HND" else (2, 1)
     sq, sk, sv, so = q.stride(), k.stride(), v.stride(), o.stride()
     if outs:
@@ -171,15 +174,17 @@ def whole_call(fn, what, q, k, v, o, layout, dims, mul, causal, pv_mode=0, q_sub
         ptrs += [t.stride(i) if t is not None else 0 for t in (outs[0], outs[2]) for i in (0, h, n)]
     else:
         ptrs = _NO_OUTS
-    call = bytearray(_CALL.pack(
-        _CALL.size, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), 0, 0, sq[0], sq[h], sq[n], sk[0], sk[h],
-        sk[n], sv[0], sv[h], sv[n], so[0], so[h], so[n], *dims, mul, _TORCH_CODES[q.dtype], int(bool(causal)),
-        pv_mode, q_sub, smooth_k, fuse_q, *ptrs))
-    nbytes = getattr(lib, what + "_workspace_bytes")(bytes(call))
+    call = _CALL.pack(
+        _CALL_SIZE, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), 0, 0, sq[0], sq[h], sq[n], sk[0], sk[h],
+        sk[n], sv[0], sv[h], sv[n], so[0], so[h], so[n], *dims, mul, _TORCH_CODES[q.dtype], 1 if causal else 0,
+        pv_mode, q_sub, smooth_k, fuse_q, *ptrs)
+    device = q.device
+    nbytes = fn_bytes(call)
     if nbytes:
-        ws = torch.empty((nbytes,), dtype=torch.uint8, device=q.device)
-        _CALL_WS.pack_into(call, _CALL_WS_AT, ws.data_ptr(), nbytes)
-    _check(fn(bytes(call), _stream(q.device)), what)
+        ws = torch.empty((nbytes,), dtype=torch.uint8, device=device)
+        call = call[:_CALL_WS_AT] + _CALL_WS.pack(ws.data_ptr(), nbytes) + call[_CALL_WS_AT + _CALL_WS.size:]
+    if fn(call, _raw_stream(device.index)):
+        _check(1, what)
 
 
 _NO_OUTS = (0,) * 12
@@ -195,8 +200,12 @@ def _on_tensor_device(fn):
     """
     @functools.wraps(fn)
     def wrapper(*args, **kwargs):
-        dev = next((a.device for a in args if isinstance(a, torch.Tensor)), None)
+        dev = args[0].device if args and isinstance(args[0], torch.Tensor) else None
+        if dev is None:
+            dev = next((a.device for a in args if isinstance(a, torch.Tensor)), None)
         if dev is None or dev.type != "cuda":
+            return fn(*args, **kwargs)
+        if torch.cuda.current_device() == dev.index:  # (nothing to switch and restore)
             return fn(*args, **kwargs)
         with torch.cuda.device(dev):
             return fn(*args, **kwargs)
@@ -204,6 +213,21 @@ def _on_tensor_device(fn):
 
 
 def _check_inputs(q, k, v, layout):
+    """(B, Hq, Hkv, Nq, Nkv, D), or the error that names what is wrong."""
+    try:
+        dims = _dims(q, layout) + _dims(k, layout)
+        B, Hq, Nq, D, Bk, Hkv, Nkv, Dk = dims
+        if (q.is_cuda and k.is_cuda and v.is_cuda and q.get_device() == k.get_device() == v.get_device()
+                and q.dtype is k.dtype is v.dtype and q.dtype in _TORCH_CODES and k.shape == v.shape
+                and B == Bk and D == Dk and q.stride(3) == 1 and k.stride(3) == 1 and v.stride(3) == 1
+                and Hkv and Hq % Hkv == 0):
+            return B, Hq, Hkv, Nq, Nkv, D
+    except (AttributeError, ValueError, IndexError):
+        pass
+    return _check_inputs_one_by_one(q, k, v, layout)
+
+
+def _check_inputs_one_by_one(q, k, v, layout):
     for name, t in (("q", q), ("k", k), ("v", v)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"sage_attn hip: invalid argument: {name} is not a tensor")
@@ -486,6 +510,6 @@ def run(q, k, v, causal=False, sm_scale=None, *, pv_dtype="fp16", q_gran="block"
         if fuse_q and pre["q8"].stride() != q.stride():
             raise ValueError("sage_attn hip: invalid argument: q8_out must be int8 with q's strides")
         outs = [pre.get(key) for key in ("q8", "q_scale", "k8", "k_scale", "km", "v_scale")]
-    whole_call(lib.sage_run, "sage_run", q, k, v, o, tensor_layout, dims, mul, causal, PV_MODES[pv_dtype], q_sub,
+    whole_call(lib.sage_run, lib.sage_run_workspace_bytes, "sage_run", q, k, v, o, tensor_layout, dims, mul, causal, PV_MODES[pv_dtype], q_sub,
                int(bool(smooth_k)), -1 if fuse_q is None else int(bool(fuse_q)), outs)
     return (o, pre) if return_intermediates else o
