@@ -25,9 +25,9 @@ struct AttnPlan {
 // 256 slots (8 waves) or 512 (4 waves, two to a CU) in rounds, a round costs
 // its start (Q, first tiles, epilogue) plus a time per 64-key block; the
 // partial kernels add the merge and its traffic.  The constants are fitted to
-// 180 shapes (both packs, 1 to 25000 rows and keys, up to 14 launches each):
-// the pick is 1.2 % slower than the best launch of each shape on average and
-// 12 % at worst, where 8 waves without a split would be 54 % on average.
+// 285 shapes (both packs, 1 to 25000 rows and keys, up to 14 launches each):
+// the pick is 1.1 % slower than the best launch of each shape on average and
+// 19 % at worst, where 8 waves without a split would be 35 % on average.
 // What they stand for: 8 waves share every tile, which is worth 18 % per
 // block on a full chip at INT8 D = 128 (B4 H32 N4096: 931 us against 958);
 // 4 waves overlap one work-group's start with another's blocks and cut
@@ -36,11 +36,11 @@ struct AttnPlan {
 // row, 4 heads to a KV head, 8192 keys: 52 us against 146).
 static AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nkv, int64_t D, bool causal,
                           bool i8, int pv_mode, int dtype, bool may_split) {
-  const double start8 = 5.5, start4 = 4.0, split_us = 3.6, merge_bytes_per_us = 7.4e6;
-  double blk8 = 0.48, blk4 = 0.46;
+  const double start8 = 5.2, start4 = 3.7, split_us = 4.2, merge_bytes_per_us = 7.4e6;
+  double blk8 = i8 ? 0.50 : 0.48, blk4 = i8 ? 0.505 : 0.525;  // D = 64
   if (D == 128) {
-    blk8 = !i8 ? 0.955 : pv_mode == SAGE_PV_F16 ? 0.61 : pv_mode == SAGE_PV_BF16 ? 0.75 : 0.60;
-    blk4 = !i8 ? 1.0 : pv_mode == SAGE_PV_FP8 ? 0.615 : 0.73;
+    blk8 = !i8 ? 0.98 : pv_mode == SAGE_PV_F16 ? 0.64 : pv_mode == SAGE_PV_BF16 ? 0.90 : 0.565;
+    blk4 = !i8 ? 1.02 : pv_mode == SAGE_PV_FP8 ? 0.58 : 0.73;
   }
   const int64_t nt = (Nkv + 63) / 64, G = Hq / Hkv;
   // blocks of a work-group: all of them, or with causal rows over several rounds the mean
@@ -54,7 +54,9 @@ static AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_
   double t = sweep((Nq + 255) / 256 * Hq * B, 256, start8, blk8, 1);
   auto consider = [&](int grp, int nsplit) {
     const bool part = grp > 1 || nsplit > 1;
-    double c = sweep((grp * Nq + 127) / 128 * (Hq / grp) * B * nsplit, 512, start4, blk4, nsplit);
+    const int64_t wgs = (grp * Nq + 127) / 128 * (Hq / grp) * B * nsplit;
+    // (a work-group that has its CU to itself takes 0.8 of a block's time)
+    double c = sweep(wgs, 512, start4, wgs <= 256 ? 0.8 * blk4 : blk4, nsplit);
     if (part) c += split_us + (double)(B * Hq * Nq * nsplit * D * 8) / merge_bytes_per_us;
     if (c < t) {
       t = c;
@@ -71,7 +73,7 @@ static AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_
     // the second S buffer (168 VGPRs): a block takes 1.5x (INT8) to 1.7x as
     // long, shared by three.  226 keys: 267 us -> 215 per call (B2 H48
     // N17776), 697 keys 110 -> 99 (B3 H12 N10198); at 8070 keys 571 -> 620.
-    const double c = sweep((Nq + 127) / 128 * Hq * B, 768, start4, i8 ? 0.71 : 0.85, 1);
+    const double c = sweep((Nq + 127) / 128 * Hq * B, 768, start4, i8 ? 0.78 : 0.90, 1);
     if (c < t) {
       t = c;
       best.nw = 4;
