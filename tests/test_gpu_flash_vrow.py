@@ -81,3 +81,23 @@ def test_far_apart_rows_take_the_tile_path(gpu_device):
     got = F.run(q, k, v)
     torch.cuda.synchronize()
     assert torch.equal(got, F.run(q, k, v.contiguous()))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Nq,Nkv", [(1, 3, 1000), (1, 65, 65), (24, 300, 257)])
+def test_infinite_last_v_row_stays_infinite(D, dtype, B, Nq, Nkv, hip_impl, gpu_device):
+    """The keys that pad the last block weigh 0 times 0, not 0 times the last
+    row's infinity: its channels are infinite and the others as without it."""
+    print(f"[vrow inf] D{D} {dtype} {B}/{Nq}/{Nkv}", flush=True)
+    g = torch.Generator().manual_seed(Nkv)
+    q, k, v = (torch.randn(B, 4, n, D, generator=g).to(dtype).to(gpu_device) for n in (Nq, Nkv, Nkv))
+    vi = v.clone()
+    vi[:, :, -1, 5] = float("inf")
+    vi[:, :, -1, 40] = float("-inf")
+    pv = "fp16" if dtype == torch.float16 else "bf16"
+    for run in (_flash().run, lambda *t: hip_impl.run(*t, pv_dtype=pv)):
+        want, got = run(q, k, v).clone(), run(q, k, vi)
+        want[..., 5], want[..., 40] = float("inf"), float("-inf")
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)

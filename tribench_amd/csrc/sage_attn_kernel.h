@@ -267,6 +267,8 @@ typedef __attribute__((address_space(3))) void lmem_t;
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4s ltr_t;
 
+static __device__ const v4i kZero16 = {0, 0, 0, 0};  // the rows of V past Nkv
+
 __device__ __forceinline__ v4i lds_read16(const char* p) { return *reinterpret_cast<const v4i*>(p); }
 // (an alias scope of its own, from __restrict__: without it the compiler
 // drains every direct-to-LDS load in flight before the read)
@@ -487,12 +489,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WP
   // ---- tile loads.  Wave load g = wave + NW*i of a K (V) tile is the 1 KB LDS
   // range [1024g, 1024g + 1024) of its slot; lane l brings the 16-byte chunk
   // that lands at offset 16l, i.e. the logical chunk (physical chunk ^ swizzle
-  // of its row).  K rows past Nkv read the last row (their P is 0), rows of V
-  // read in place too (P = 0 meets a value that the block holds anyway); V
-  // tiles are zero past Nkv.  Loads past the tile go to the sink, so every
-  // wave issues KPW loads per K tile and VPW per V tile.  `whole`: every row
-  // of the tile is < Nkv, so each load is a uniform tile base plus a lane
-  // offset that does not change from tile to tile.
+  // of its row).  K rows past Nkv read the last row (their P is 0); V rows past
+  // Nkv are zero, in the V tiles and read in place (kZero16: the last row
+  // again would make 0 * inf of an infinity in it).  Loads past the tile go to
+  // the sink, so every wave issues KPW loads per K tile and VPW per V tile.
+  // `whole`: every row of the tile is < Nkv, so each load is a uniform tile
+  // base plus a lane offset that does not change from tile to tile.
   uint32_t kfoff[KPW], vfoff[VPW];
 #pragma unroll
   for (int i = 0; i < KPW; ++i) {
@@ -505,7 +507,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WP
     const int p = 64 * (wave + NW * i) + lane;
     if constexpr (kVRow) {
       const int r = p / (2 * D / 16), pc = p % (2 * D / 16);
-      vfoff[i] = wave + NW * i < VLD ? (uint32_t)(r * a.svn * EB + 16 * (pc ^ vrow_swz<D>(r))) : 0u;
+      vfoff[i] = wave + NW * i < VLD ? (uint32_t)r * a.svn * EB + (uint32_t)(16 * (pc ^ vrow_swz<D>(r))) : 0u;
     } else {
       const int d = p / (VRB / 16), pc = p % (VRB / 16);
       vfoff[i] = wave + NW * i < VLD ? (uint32_t)(d * VRB + 16 * (pc ^ swz<VRB>(d))) : 0u;
@@ -543,8 +545,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WP
       const char* src = in ? base + vfoff[i] : kbase;
       if (kVRow && !whole && in) {
         const int p = 64 * g + lane;
-        const int r = p / (2 * D / 16), pc = p % (2 * D / 16);
-        src = base + (uint32_t)(min(r, nkv - 1 - j * kBN) * a.svn * EB + 16 * (pc ^ vrow_swz<D>(r)));
+        const int r = p / (2 * D / 16);
+        src = r < nkv - j * kBN ? base + vfoff[i] : reinterpret_cast<const char*>(&kZero16);
       }
       char* dst = in ? slot + 1024 * g : smem + RING;
       __builtin_amdgcn_global_load_lds((gmem_t*)src, (lmem_t*)dst, 16, 0, 0);
