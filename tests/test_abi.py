@@ -229,3 +229,35 @@ def test_attn_fwd_q_rejects_bad_arguments(lib):
         rc = lib.sage_attn_fwd_q(*a.values())
         msg = lib.sage_last_error().decode()
         assert rc != 0 and "invalid argument" in msg and needle in msg, msg
+
+
+def _sage_call(hip_impl, **over):
+    """A packed sage_call of one 64-row head; every buffer at address 256."""
+    c = dict(B=1, Hq=1, Hkv=1, Nq=64, Nkv=64, D=128, mul=0.1, dtype=2, fuse_q=-1, q_row=128, ws=1 << 40)
+    c.update(over)
+    rows = [64 * 128, 64 * 128, 128]
+    return hip_impl._CALL.pack(hip_impl._CALL_SIZE, 256, 256, 256, 256, 256, c["ws"], rows[0], rows[1], c["q_row"],
+                               *rows, *rows, *rows, c["B"], c["Hq"], c["Hkv"], c["Nq"], c["Nkv"], c["D"], c["mul"],
+                               c["dtype"], 0, 0, 128, 1, c["fuse_q"], *hip_impl._NO_OUTS)
+
+
+@pytest.mark.parametrize("Hq", [1, 512])  # by size, Q is quantized in the pre-pass or in the prologue
+def test_sage_run_limits_do_not_depend_on_the_shape(lib, hip_impl, Hq):
+    import torch
+
+    for over, needle in [
+        (dict(mul=0.0), "mul"),
+        (dict(mul=-1.0), "mul"),
+        (dict(mul=float("inf")), "mul"),
+        (dict(mul=-1.0, D=64, fuse_q=1), "mul"),
+        (dict(q_row=1 << 25), "2^31 bytes"),
+    ]:
+        assert lib.sage_run(_sage_call(hip_impl, Hq=Hq, **over), None) != 0
+        msg = lib.sage_last_error().decode()
+        assert "invalid argument" in msg and needle in msg, msg
+    if torch.cuda.is_available():  # what is not refused would launch on these addresses
+        return
+    for over in [dict(mul=-1.0, D=64), dict(mul=-1.0, fuse_q=0), dict(q_row=1 << 25, D=64)]:
+        assert lib.sage_run(_sage_call(hip_impl, Hq=Hq, **over), None) != 0  # no device: the launch fails
+        msg = lib.sage_last_error().decode()
+        assert "invalid argument" not in msg, msg

@@ -380,6 +380,14 @@ static int attn_args(AttnArgs& a, const char* who, const sage_call& c, bool quan
   return 0;
 }
 
+// Q the attention's prologue can quantize: a positive finite multiplier, a
+// head's rows within 2^31 bytes (32-bit row offsets).
+static bool q_fusable(const sage_call& c) {
+  const float mul = (float)c.mul;
+  const int qes = c.dtype == SAGE_DTYPE_F32 ? 4 : 2;
+  return mul > 0.0f && mul != INFINITY && (c.Nq * c.q_strides[2] + c.D) * qes < 0x7FFFFFFF;
+}
+
 // Stages of one sage_run call and the pieces of its workspace.
 struct RunPlan {
   AttnPlan attn;
@@ -398,7 +406,8 @@ static RunPlan run_plan(const sage_call* c) {
   // faster per call (226 keys, B2 H48 N17776 D64: 267 us against 292), with
   // fewer the start is what counts and the pre-pass is 1 to 9 % faster (B1 H18
   // N159 D128: 24.6 us against 26.8).
-  r.fuse_q = c->fuse_q < 0 ? (c->Nq + 127) / 128 * c->Hq * c->B > 256 : c->fuse_q != 0;
+  // (the prologue takes only what sage_attn_fwd_q does: q_fusable)
+  r.fuse_q = c->fuse_q < 0 ? (c->Nq + 127) / 128 * c->Hq * c->B > 256 && q_fusable(*c) : c->fuse_q != 0;
   r.quant_q = !r.fuse_q || r.attn.part();  // the partial kernels read Q8
   // V already in the P.V type: read in place, no V tiles (4 bytes of traffic
   // per element less: fp16 B8 H16 N4096 D64 548 us -> 536, 32 rows over 16384
@@ -465,7 +474,12 @@ extern "C" int sage_run(const sage_call* c, void* stream) {
   float* km = static_cast<float*>(c->smooth_k ? (c->km ? c->km : ws + r.off_km) : nullptr);
   float* vs = static_cast<float*>(r.v_mode != SAGE_V_NONE ? (c->v_scale ? c->v_scale : ws + r.off_vs) : nullptr);
   const float mul = (float)c->mul;
-  if (r.fuse_q && (!(mul > 0.0f) || mul == INFINITY)) return fail("%s: invalid argument: mul %g", who, mul);
+  // A call is held to the prologue's limits by its options (left to choose, by
+  // the head dim), not by where its shape has Q quantized.
+  if ((c->fuse_q < 0 ? c->D == 128 : c->fuse_q != 0) && !q_fusable(*c)) {
+    if (!(mul > 0.0f) || mul == INFINITY) return fail("%s: invalid argument: mul %g", who, mul);
+    return fail("%s: invalid argument: a head's rows must span < 2^31 bytes", who);
+  }
 
   const int pv = (int)c->pv_mode, dt = (int)c->dtype, q_sub = (int)c->q_sub;
   const bool dq = r.quant_q;
