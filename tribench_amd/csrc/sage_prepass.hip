@@ -262,14 +262,21 @@ __device__ __forceinline__ void kstats_chunk(const T* __restrict__ ksrc, int64_t
     acc[e] = 0.0f;
     vm[e] = 0.0f;
   }
-  constexpr int U = 4;  // rows in flight per thread
+  // Rows in flight per thread: the 256 rows of the smallest chunk (D = 128:
+  // 16 of 16 bytes; fp32 half of them, 64 VGPRs of loads either way).  There
+  // are at most 16 chunks to a head, so a few heads leave a block to a CU and
+  // its time is the number of load latencies in a row: whole calls 78.8 ->
+  // 76.8 us against 4 rows in flight at B2 Hkv8 N16384 D128, 49.6 -> 49.1 at
+  // B1 H24 N1333, the larger ones even.
+  constexpr int U = sizeof(T) == 4 && TL == 16 ? 8 : 256 / TL;
+  auto load_rows = [&](Raw8<T> (&r)[U], const T* src, int64_t sn, int64_t nb) __attribute__((always_inline)) {
+    // (rows past the chunk read its last one and are left out below)
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u] = load8<T>(src + min<int64_t>(nb + (int64_t)u * TL, n1 - 1) * sn + cg * 8);
+  };
   for (int64_t nb = n0 + tl; nb < n1; nb += (int64_t)TL * U) {
     Raw8<T> r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t n = nb + (int64_t)u * TL;
-      r[u] = (n < n1) ? load8<T>(ksrc + n * ksn + cg * 8) : zero8<T>();
-    }
+    load_rows(r, ksrc, ksn, nb);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (nb + (int64_t)u * TL < n1) {
@@ -278,11 +285,7 @@ __device__ __forceinline__ void kstats_chunk(const T* __restrict__ ksrc, int64_t
       }
     }
     if (vsrc) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t n = nb + (int64_t)u * TL;
-        r[u] = (n < n1) ? load8<T>(vsrc + n * vsn + cg * 8) : zero8<T>();
-      }
+      load_rows(r, vsrc, vsn, nb);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
 #pragma unroll
@@ -290,41 +293,31 @@ __device__ __forceinline__ void kstats_chunk(const T* __restrict__ ksrc, int64_t
       }
     }
   }
-  // tree over the TL token lanes: acc[tl] += acc[tl + s], s = TL/2 .. 1.
-  // Row r of red_s holds channel group cg's values 0-3 and 4-7 as 16-byte
-  // units cg and CG + cg, swapped in odd rows, so that the units a wave
-  // writes or reads together never share a bank.
-  auto at = [&](int r, int e) { return red_s + r * D + 4 * (cg + CG * ((e >> 2) ^ (r & 1))) + (e & 3); };
+  // tree over the TL token lanes: acc[tl] += acc[tl + s], s = TL/2 .. 1, by one
+  // thread per channel in registers (a barrier per step took longer).  Row r
+  // of red_s holds channel group cg's values 0-3 and 4-7 as 16-byte units cg
+  // and CG + cg, swapped in odd rows, so that the units a wave writes
+  // together never share a bank.
+  auto at = [&](int r, int g, int e) { return red_s + r * D + 4 * (g + CG * ((e >> 2) ^ (r & 1))) + (e & 3); };
+  auto tree = [&](const float (&x)[8], float* out, auto op) __attribute__((always_inline)) {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) *at(tl, e) = acc[e];
-  __syncthreads();
-  for (int s = TL / 2; s >= 1; s >>= 1) {
-    if (tl < s) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) *at(tl, e) = *at(tl, e) + *at(tl + s, e);
-    }
+    for (int e = 0; e < 8; ++e) *at(tl, cg, e) = x[e];
     __syncthreads();
-  }
-  if (psum && tl == 0) {  // (no K smoothing: FP8 V statistics only, no sums)
+    if (tid < D) {
+      float v[TL];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) psum[cg * 8 + e] = *at(0, e);
-  }
+      for (int t = 0; t < TL; ++t) v[t] = *at(t, tid >> 3, tid & 7);
+#pragma unroll
+      for (int s = TL / 2; s >= 1; s >>= 1)
+#pragma unroll
+        for (int t = 0; t < s; ++t) v[t] = op(v[t], v[t + s]);
+      out[tid] = v[0];
+    }
+  };
+  if (psum) tree(acc, psum, [](float a, float b) { return a + b; });  // (no K smoothing: FP8 V statistics only)
   if (vsrc) {
     __syncthreads();
-#pragma unroll
-    for (int e = 0; e < 8; ++e) *at(tl, e) = vm[e];
-    __syncthreads();
-    for (int s = TL / 2; s >= 1; s >>= 1) {
-      if (tl < s) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) *at(tl, e) = fmaxf(*at(tl, e), *at(tl + s, e));
-      }
-      __syncthreads();
-    }
-    if (tl == 0) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) pamax[cg * 8 + e] = *at(0, e);
-    }
+    tree(vm, pamax, [](float a, float b) { return fmaxf(a, b); });
   }
 }
 
