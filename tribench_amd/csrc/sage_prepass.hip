@@ -54,6 +54,7 @@ struct PrepassArgs {
   int64_t nqb, nkb;  // blocks per head
   int64_t n_stat, n_qblk_a, n_kblk_a;  // role counts of launch A
   int64_t n_kblk_b, n_qblk_b;          // role counts of launch B (K blocks first)
+  int k_waves;                         // launch B's K roles are quant_k_waves
   uint8_t* vt;                         // V tiles (sage_prepass_vt), else NULL
   int pv_mode;                         // their type
   int64_t ntile;                       // 64-key tiles per head
@@ -248,7 +249,13 @@ __device__ __forceinline__ void quant_block(const T* __restrict__ src, int64_t s
 // sage_quant_math.h (if psum: K smoothing), and (if vsrc) channel max|v|.
 // At least one of psum and vsrc is non-null.
 // ---------------------------------------------------------------------------
-template <typename T, int D>
+// U: rows in flight per thread.  There are at most 16 chunks to a head, so a few
+// heads leave a block to a CU and its time is the number of load latencies in a
+// row: 8 rows where the launch has no V tiles (pre-pass 15.3 -> 13.6 us at B2
+// Hkv12 N1500 D64, 27.4 -> 24.0 at B1 Hkv3 N9000 D128, both FP8 V), 4 beside V
+// tiles, which lack waves with the VGPRs of 8 (22.6 us -> 25.1 at B4 Hkv8 N2300
+// D128).
+template <typename T, int D, int U>
 __device__ __forceinline__ void kstats_chunk(const T* __restrict__ ksrc, int64_t ksn, const T* __restrict__ vsrc,
                              int64_t vsn, int64_t n0, int64_t n1, float* __restrict__ psum,
                              float* __restrict__ pamax, float* red_s) {
@@ -262,17 +269,16 @@ __device__ __forceinline__ void kstats_chunk(const T* __restrict__ ksrc, int64_t
     acc[e] = 0.0f;
     vm[e] = 0.0f;
   }
-  // Rows in flight per thread: the 256 rows of the smallest chunk (D = 128:
-  // 16 of 16 bytes; fp32 half of them, 64 VGPRs of loads either way).  There
-  // are at most 16 chunks to a head, so a few heads leave a block to a CU and
-  // its time is the number of load latencies in a row: whole calls 78.8 ->
-  // 76.8 us against 4 rows in flight at B2 Hkv8 N16384 D128, 49.6 -> 49.1 at
-  // B1 H24 N1333, the larger ones even.
-  constexpr int U = sizeof(T) == 4 && TL == 16 ? 8 : 256 / TL;
   auto load_rows = [&](Raw8<T> (&r)[U], const T* src, int64_t sn, int64_t nb) __attribute__((always_inline)) {
-    // (rows past the chunk read its last one and are left out below)
+    // (rows past the chunk are left out below: zero, or with 8 in flight its
+    // last row again, without a branch; with 4 the branch is the cheaper,
+    // 30.5 us against 36.7 for the pre-pass at B1 Hkv1 N30000 D128)
 #pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = load8<T>(src + min<int64_t>(nb + (int64_t)u * TL, n1 - 1) * sn + cg * 8);
+    for (int u = 0; u < U; ++u) {
+      const int64_t n = nb + (int64_t)u * TL;
+      if constexpr (U == 4) r[u] = n < n1 ? load8<T>(src + n * sn + cg * 8) : zero8<T>();
+      else r[u] = load8<T>(src + min(n, n1 - 1) * sn + cg * 8);
+    }
   };
   for (int64_t nb = n0 + tl; nb < n1; nb += (int64_t)TL * U) {
     Raw8<T> r[U];
@@ -404,13 +410,14 @@ __device__ __forceinline__ void quant_k_role(const PrepassArgs& a, int64_t r, co
 }
 
 // NIQ / NIK: 16-element items per thread of a Q / K block (blk * D / 4096).
-template <typename T, int D, int NIQ, int NIK>
+// kVt: the launch has V tiles.
+template <typename T, int D, int NIQ, int NIK, bool kVt>
 __global__ __launch_bounds__(kPrepassThreads) void prepass_a_kernel(PrepassArgs a) {
   __shared__ uint32_t amax_s[16];
   __shared__ float scl_s[16], rcp_s[16];
   // one pool for the statistics' reduction rows or a V tile's transpose
   constexpr int kRed = kPrepassThreads / (D / 8) * D * (int)sizeof(float);
-  __shared__ __attribute__((aligned(16))) char pool[kRed > vtile_pool_bytes<D>() ? kRed : vtile_pool_bytes<D>()];
+  __shared__ __attribute__((aligned(16))) char pool[!kVt || kRed > vtile_pool_bytes<D>() ? kRed : vtile_pool_bytes<D>()];
   float* red_s = reinterpret_cast<float*>(pool);
   int64_t r = blockIdx.x;
   if (r < a.n_stat) {
@@ -420,7 +427,7 @@ __global__ __launch_bounds__(kPrepassThreads) void prepass_a_kernel(PrepassArgs 
     const T* vs = a.v_fp8 ? static_cast<const T*>(a.v) + b * a.sv[0] + h * a.sv[1] : nullptr;
     const int64_t slot = ((b * a.Hkv + h) * a.nch + c) * D;
     // psum is NULL without K smoothing (the workspace then holds the V maxima only)
-    kstats_chunk<T, D>(ks, a.sk[2], vs, a.sv[2], n0, n1, a.smooth_k ? a.psum + slot : nullptr,
+    kstats_chunk<T, D, kVt ? 4 : 8>(ks, a.sk[2], vs, a.sv[2], n0, n1, a.smooth_k ? a.psum + slot : nullptr,
                        a.v_fp8 ? a.pamax + slot : nullptr, red_s);
     return;
   }
@@ -435,7 +442,8 @@ __global__ __launch_bounds__(kPrepassThreads) void prepass_a_kernel(PrepassArgs 
     return;
   }
   r -= a.n_kblk_a;
-  if (r < a.n_vt_a) vtile_role<T, D>(a, r, nullptr, pool);  // fp16 / bf16 tiles
+  if constexpr (kVt)
+    if (r < a.n_vt_a) vtile_role<T, D>(a, r, nullptr, pool);  // fp16 / bf16 tiles
 }
 
 // Channel mean of K (km_s) and FP8 V scale (vs_s, unless null) of one
@@ -471,8 +479,74 @@ __device__ __forceinline__ void head_stats(const PrepassArgs& a, int64_t b, int6
   }
 }
 
+// Four K blocks of one head, one to each wave: 16-bit K in blocks of 64 rows.
+// A wave holds its whole block (64 rows x D, 64 or 128 bytes per lane and 32
+// rows), so the block's max is a wave reduction, without the barriers and
+// LDS atomics of quant_block, four blocks share the head's statistics, and
+// four times the bytes are in flight.  Same arithmetic, same bits.  K of B8
+// H32 N4096 D128 (0.40 GB read and written): 107 us -> 87, 4.6 TB/s.
+// Lane l holds channels 16(l % CPR) .. +16 of rows l / CPR + (64 / CPR) j.
+template <typename T, int D>
+__device__ __forceinline__ void quant_k_waves(const PrepassArgs& a, int64_t r, float* km_s, float* vs_s) {
+  constexpr int CPR = D / 16, RPI = 64 / CPR, NJ = 64 / RPI;
+  const int lane = threadIdx.x & 63, c = lane % CPR;
+  const int64_t nkg = (a.nkb + 3) / 4, g = r % nkg, h = (r / nkg) % a.Hkv, b = r / (nkg * a.Hkv);
+  const int64_t kb = 4 * g + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row0 = min(kb, a.nkb - 1) * 64;  // (a wave past the head's blocks loads the last one)
+  const int rows_valid = (int)min<int64_t>(64, a.Nkv - row0);
+  const T* src = static_cast<const T*>(a.k) + b * a.sk[0] + h * a.sk[1] + row0 * a.sk[2] + 16 * c;
+  Raw8<T> raw[NJ][2];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {  // rows past Nkv repeat the last one: the max is the same, no store
+    const T* p = src + min(lane / CPR + RPI * j, rows_valid - 1) * a.sk[2];
+    raw[j][0] = load8<T>(p);
+    raw[j][1] = load8<T>(p + 8);
+  }
+  head_stats<D>(a, b, h, g == 0, km_s, g == 0 ? vs_s : nullptr);
+  __syncthreads();
+  if (kb >= a.nkb) return;
+  float kmr[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) kmr[e] = a.smooth_k ? km_s[stat_slot(16 * c + e)] : 0.0f;
+  float am = 0.0f;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) am = fmaxf(am, fabsf(elem<T>(raw[j][e >> 3], e & 7) - kmr[e]));
+  const float sc = block_scale(__uint_as_float(wave_max_u32(__float_as_uint(am))));
+  const float rc = sc > 0.0f ? 1.0f / sc : 0.0f;
+  if (lane == 0) a.k_scale[(b * a.Hkv + h) * a.nkb + kb] = sc;
+  // (the smoothed values are formed again below: kept from the max, they take
+  // 128 VGPRs and halve the waves in flight)
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      uint4& u = raw[j][i].u[0];
+      asm("" : "+v"(u.x), "+v"(u.y), "+v"(u.z), "+v"(u.w));
+    }
+  int8_t* dst = a.k8 + b * a.sk8[0] + h * a.sk8[1] + row0 * a.sk8[2] + 16 * c;
+  auto quantize = [&](auto fast_tag) __attribute__((always_inline)) {
+    constexpr bool kFast = decltype(fast_tag)::value;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int row = lane / CPR + RPI * j;
+      uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        w[e >> 2] |= (uint32_t)(uint8_t)quant_elem(elem<T>(raw[j][e >> 3], e & 7) - kmr[e], sc, rc, kFast)
+                     << (8 * (e & 3));
+      if (row < rows_valid) *reinterpret_cast<uint4*>(dst + row * a.sk8[2]) = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  };
+  if (fast_div_ok(sc)) quantize(std::true_type{});
+  else quantize(std::false_type{});
+}
+
 // Roles: K blocks, then Q blocks, then (FP8 P.V) V tiles.
-template <typename T, int D, int NIQ, int NIK>
+// kWaves: the K roles are quant_k_waves (a kernel of its own: with its 108 VGPRs
+// at D = 128 the other K role would have 4 work-groups to a CU instead of 7).
+template <typename T, int D, int NIQ, int NIK, bool kWaves>
 __global__ __launch_bounds__(kPrepassThreads) void prepass_b_kernel(PrepassArgs a) {
   __shared__ uint32_t amax_s[16];
   __shared__ float scl_s[16], rcp_s[16];
@@ -489,6 +563,10 @@ __global__ __launch_bounds__(kPrepassThreads) void prepass_b_kernel(PrepassArgs 
   }
   if (r >= a.n_kblk_b) {
     quant_q_role<T, D, NIQ>(a, r - a.n_kblk_b, amax_s, scl_s, rcp_s);
+    return;
+  }
+  if constexpr (kWaves) {
+    quant_k_waves<T, D>(a, r, km_s, vs_s);
     return;
   }
   const int64_t kb = r % a.nkb, h = (r / a.nkb) % a.Hkv, b = r / (a.nkb * a.Hkv);
@@ -511,12 +589,20 @@ template <typename T, int D, int NIQ, int NIK>
 static int launch_prepass_ni(const PrepassArgs& a, hipStream_t st) {
   const int64_t na = a.n_stat + a.n_qblk_a + a.n_kblk_a + a.n_vt_a;
   if (na > 0) {
-    hipLaunchKernelGGL((prepass_a_kernel<T, D, NIQ, NIK>), dim3((unsigned)na), dim3(kPrepassThreads), 0, st, a);
+    if (a.n_vt_a > 0)
+      hipLaunchKernelGGL((prepass_a_kernel<T, D, NIQ, NIK, true>), dim3((unsigned)na), dim3(kPrepassThreads), 0, st, a);
+    else
+      hipLaunchKernelGGL((prepass_a_kernel<T, D, NIQ, NIK, false>), dim3((unsigned)na), dim3(kPrepassThreads), 0, st, a);
     if (int rc = check_launch("sage_prepass (launch A)")) return rc;
   }
   if (a.n_kblk_b > 0) {
     const int64_t nb = a.n_kblk_b + a.n_qblk_b + a.n_vt_b;
-    hipLaunchKernelGGL((prepass_b_kernel<T, D, NIQ, NIK>), dim3((unsigned)nb), dim3(kPrepassThreads), 0, st, a);
+    if constexpr (sizeof(T) == 2 && NIK == 64 * D / 4096)
+      if (a.k_waves) {
+        hipLaunchKernelGGL((prepass_b_kernel<T, D, NIQ, NIK, true>), dim3((unsigned)nb), dim3(kPrepassThreads), 0, st, a);
+        return check_launch("sage_prepass (launch B)");
+      }
+    hipLaunchKernelGGL((prepass_b_kernel<T, D, NIQ, NIK, false>), dim3((unsigned)nb), dim3(kPrepassThreads), 0, st, a);
     if (int rc = check_launch("sage_prepass (launch B)")) return rc;
   }
   return 0;
@@ -652,7 +738,6 @@ int sage::prepass_any(const char* who, const void* q, const void* k, const void*
   a.n_stat = need_b ? a.nch * Hkv * B : 0;
   a.n_qblk_a = need_b || !do_q ? 0 : a.nqb * Hq * B;
   a.n_kblk_a = need_b ? 0 : a.nkb * Hkv * B;
-  a.n_kblk_b = need_b ? a.nkb * Hkv * B : 0;
   a.n_qblk_b = need_b && do_q ? a.nqb * Hq * B : 0;
   // V tiles last in their launch: B for FP8 (they need v_scale), and B for
   // fp16/bf16 too when B quantizes only K (its VALU-bound K blocks then share
@@ -663,6 +748,16 @@ int sage::prepass_any(const char* who, const void* q, const void* k, const void*
   const bool vt_in_b = vt && (pv_mode == SAGE_PV_FP8 || (need_b && !do_q));
   a.n_vt_a = vt && !vt_in_b ? a.ntile * Hkv * B : 0;
   a.n_vt_b = vt_in_b ? a.ntile * Hkv * B : 0;
+  // A wave to a K block needs 4 blocks to a CU to pay beside V tiles, 8 without
+  // (that launch is bound by the role's latency, which is longer).  bf16,
+  // with fp16 V tiles, D = 128: 512 blocks 13.6 us against 14.8, 1024 21.7 ->
+  // 17.9, 4096 58 -> 53, 16384 252 -> 227; D = 64: 9.2 against 9.7, 13.5 -> 10.7,
+  // 32.5 -> 28.3, 120 -> 112.  Without them here: 1136 blocks 14.7 against 15.5 at
+  // D = 64, 1152 25.5 against 26.9 at 128; 2048 15.4 -> 11.5 and 25.8 -> 19.8.  (fp32
+  // would take 128 VGPRs for its loads alone and runs at 5.9 TB/s without.)
+  a.k_waves = need_b && in_dtype != SAGE_DTYPE_F32 && blkq == 128 && blkk == 64 && !vrows &&
+              a.nkb * Hkv * B >= (vt_in_b ? 1024 : 2048);
+  a.n_kblk_b = need_b ? (a.k_waves ? (a.nkb + 3) / 4 : a.nkb) * Hkv * B : 0;
   if (a.n_stat + a.n_qblk_a + a.n_kblk_a + a.n_vt_a > 0x7FFFFFFF || a.n_kblk_b + a.n_qblk_b + a.n_vt_b > 0x7FFFFFFF)
     return fail("%s: invalid argument: grid too large", who);
 
