@@ -9,8 +9,9 @@ stream:
 
     sage_prepass     per_block_int8 (triton_impl.py:35-82) + K smoothing (+ FP8 V scales)
     sage_vtiles      v.to(torch.float16) (triton_impl.py:189), in the attention's V tile layout
-    sage_prepass_vt  both, in the pre-pass's launches (what run() uses)
+    sage_prepass_vt  both, in the pre-pass's launches
     sage_attn_fwd    _attn_fwd launch (triton_impl.py:186-199); sage_attn_fwd_q quantizes Q itself
+    sage_run         the whole call with launches chosen by its shape (what run() uses)
 
 There is no CPU or PyTorch fallback: without a ROCm device or without the
 library the call raises.  The module is loaded by file path (no parent
@@ -367,8 +368,8 @@ def q_sub_of(q_gran):
 
 
 def fuse_q_default(head_dim):
-    """Where Q is quantized when the caller does not say: in the attention
-    kernel's prologue at D = 128 (measured 1-2 % faster per forward at
+    """Where the stage calls (and intermediates) have Q quantized when the caller
+    does not say: in the attention kernel's prologue at D = 128 (measured 1-2 % faster per forward at
     configurations 2 and 3, even at 5), in the pre-pass at D = 64 (the
     prologue costs more than it saves there: 2 % slower at configuration 4)."""
     return head_dim == 128
@@ -487,7 +488,7 @@ def run(q, k, v, causal=False, sm_scale=None, *, pv_dtype="fp16", q_gran="block"
     smooth_k   subtract the per-channel K mean before quantizing (default on)
     fuse_q     quantize Q in the attention kernel's prologue (True) or in the
                pre-pass (False): the same Q8 and scales bit for bit; by
-               default (None) as fuse_q_default(D) measured faster
+               default (None) the faster one for the shape
     """
     if pv_dtype not in PV_MODES:
         raise ValueError(f"sage_attn hip: invalid argument: pv_dtype {pv_dtype!r}")
