@@ -4,9 +4,11 @@
 stage entry points (``attention`` on the pre-pass's own outputs, sage_flash_fwd
 on V tiles) always sweep all keys at once.  Q8, K8 and the scales are the same;
 P is rounded to its type against another running max (e_p = 2^-11 fp16, 2^-9
-bf16, 2^-4 e4m3, relative), the row sums of fp16 P carry 5 * 2^-11 each, and O
-is rounded to its type (e_o), so
+bf16, relative), the row sums of fp16 P carry 5 * 2^-11 each, and O is rounded
+to its type (e_o), so
   |a - b| <= 2 e_p max|v| + (2 e_o + 10 * 2^-11) |o|.
+FP8 P would move by 2^-4, the type's whole error, so its keys are not split; its
+packed heads sweep the same blocks: equal bit for bit.
 Shapes: single rows, rows that fill a tile with packed heads and ones that end
 in the middle of a head, keys that leave the last range short, causal rows that
 see nothing of a range, every Q-scale granularity, both layouts.
@@ -19,7 +21,7 @@ import torch
 from test_gpu_flash_vrow import _flash, _tiles
 
 pytestmark = pytest.mark.gpu
-E = {"fp16": 2.0 ** -11, "bf16": 2.0 ** -9, "fp8": 2.0 ** -4}
+E = {"fp16": 2.0 ** -11, "bf16": 2.0 ** -9}
 DT = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
 EO = {"bf16": 2.0 ** -9, "fp16": 2.0 ** -11, "fp32": 2.0 ** -24}
 
@@ -27,6 +29,7 @@ EO = {"bf16": 2.0 ** -9, "fp16": 2.0 ** -11, "fp32": 2.0 ** -24}
 SHAPES = [(1, 1, 1, 1, 65, False), (1, 4, 1, 1, 4097, False), (2, 6, 2, 37, 3000, False),
           (3, 8, 2, 32, 1000, False), (1, 12, 3, 127, 2111, False), (1, 2, 2, 130, 5000, False),
           (1, 2, 1, 1500, 1500, True), (1, 3, 3, 777, 777, True)]
+PACKED = [(64, 32, 8, 1, 200, False), (96, 18, 3, 5, 131, False), (64, 16, 2, 3, 700, False)]  # FP8 too
 
 
 def _inputs(shape, D, dtype, dev, seed=3):
@@ -71,9 +74,33 @@ def test_int8_split_matches_one_sweep(shape, D, hip_impl, gpu_device):
         for key in ("q8", "q_scale", "k8", "k_scale", "km"):
             assert torch.equal(pre[key], stage[key]), key
         want = hip_impl.attention(q, k, v, stage, causal, pv_dtype=pv, q_sub=q_sub, tensor_layout=layout)
-        _close(o, want, v, E[pv], EO[dtype])
+        if pv == "fp8":
+            assert torch.equal(o, want)
+        else:
+            _close(o, want, v, E[pv], EO[dtype])
         fused = hip_impl.run(q, k, v, causal=causal, pv_dtype=pv, q_gran=gran, tensor_layout=layout, fuse_q=True)
         assert torch.equal(fused, o)  # where Q is quantized changes no bit
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("shape", SHAPES + PACKED, ids=lambda s: "-".join(str(int(x)) for x in s))
+def test_fp8_rows_do_not_depend_on_the_call(shape, D, hip_impl, gpu_device):
+    """FP8 P: the whole call gives one sweep's bits in every type, layout and
+    Q granularity, heads packed or not, and so does a batch entry alone."""
+    causal = shape[5]
+    for gran, dtype, layout in [("block", "bf16", "HND"), ("wave", "fp16", "NHD"), ("thread", "fp32", "HND")]:
+        print(f"[fp8 rows] {shape} D{D} {gran} {dtype} {layout}", flush=True)
+        q, k, v = _inputs(shape, D, dtype, gpu_device)
+        if layout == "NHD":
+            q, k, v = (t.transpose(1, 2).contiguous() for t in (q, k, v))
+        kw = dict(pv_dtype="fp8", tensor_layout=layout)
+        o = hip_impl.run(q, k, v, causal=causal, q_gran=gran, **kw)
+        q_sub = hip_impl.q_sub_of(gran)
+        stage = hip_impl.prepass(q, k, v, q_sub=q_sub, **kw)
+        assert torch.equal(o, hip_impl.attention(q, k, v, stage, causal, q_sub=q_sub, **kw))
+        one = hip_impl.run(*(t[-1:] for t in (q, k, v)), causal=causal, q_gran=gran, **kw)
+        torch.cuda.synchronize()
+        assert torch.equal(one, o[-1:])
 
 
 @pytest.mark.parametrize("D", [64, 128])

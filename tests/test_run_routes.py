@@ -1,0 +1,88 @@
+"""Which launches sage_run and sage_flash_run take, and with which layouts, on
+a host without a GPU: the C ABI's own source with recording stand-ins for the
+pre-pass and the kernel launches (tests/native/run_routes.cpp)."""
+from __future__ import annotations
+
+import ctypes
+import json
+import random
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from tribench_amd import build as hip_build
+
+HERE = Path(__file__).resolve().parent
+PV = {"fp16": 0, "bf16": 1, "fp8": 2}
+DT = {"fp32": 0, "fp16": 1, "bf16": 2}
+BUF, Q8 = 1 << 20, 1 << 21  # addresses nothing reads
+
+
+@pytest.fixture(scope="module")
+def routes(tmp_path_factory, hip_impl):
+    so = hip_impl.library_path()
+    out = tmp_path_factory.mktemp("routes") / "run_routes.so"
+    subprocess.run([hip_build.hipcc(), *hip_build.COMMON, "-O0", "-w", "-shared", "-x", "hip",
+                    str(HERE / "native" / "run_routes.cpp"), "-x", "none", str(so), f"-Wl,-rpath,{so.parent}",
+                    "-Wl,-Bsymbolic", "-o", str(out)], check=True, capture_output=True)
+    lib = ctypes.CDLL(str(out))
+    lib.take_routes.restype = lib.sage_last_error.restype = ctypes.c_char_p
+    for name in ("sage_run", "sage_flash_run"):
+        getattr(lib, name).argtypes = [ctypes.c_char_p, ctypes.c_void_p]
+        getattr(lib, name + "_workspace_bytes").restype = ctypes.c_size_t
+        getattr(lib, name + "_workspace_bytes").argtypes = [ctypes.c_char_p]
+    return lib
+
+
+def dense(H, N, D):
+    return [H * N * D, N * D, D]
+
+
+def run_call(lib, hip_impl, B, Hq, Hkv, Nq, Nkv, D, *, flash=False, dtype="bf16", causal=False, pv="fp16", q_sub=128,
+             smooth_k=1, fuse_q=-1, q_strides=None, outs=None, q8_strides=None, k8_strides=None):
+    """(status, routes or message) of one call with the workspace it asks for;
+    outs: addresses of q8, q_scale, k8, k_scale, km, v_scale."""
+    sq, sk = dense(Hq, Nq, D), dense(Hkv, Nkv, D)
+    name = "sage_flash_run" if flash else "sage_run"
+
+    def pack(ws, n):
+        return hip_impl._CALL.pack(hip_impl._CALL_SIZE, BUF, BUF, BUF, BUF, ws, n, *(q_strides or sq), *sk, *sk, *sq,
+                                   B, Hq, Hkv, Nq, Nkv, D, 0.1, DT[dtype], int(causal), PV[pv], q_sub, smooth_k,
+                                   fuse_q, *(outs or [0] * 6), *(q8_strides or [0] * 3), *(k8_strides or [0] * 3))
+
+    n = getattr(lib, name + "_workspace_bytes")(pack(0, 0))
+    lib.take_routes()
+    rc = getattr(lib, name)(pack(BUF if n else 0, n), None)
+    if rc:
+        return rc, lib.sage_last_error().decode()
+    return 0, [json.loads(line) for line in lib.take_routes().decode().splitlines()]
+
+
+def test_fp8_keys_stay_in_one_sweep(routes, hip_impl):
+    """FP8 P is rounded against the sweep's running max, so ranges would give
+    other codes: whatever the shape, one range; rows of few heads may still
+    share a work-group.  The same shapes with fp16 P do split."""
+    rng = random.Random(1)
+    split = packed = 0
+    for _ in range(400):
+        Hkv, G = rng.choice([1, 2, 3, 8, 16]), rng.choice([1, 2, 4, 6])
+        shape = (rng.choice([1, 2, 8, 64, 200]), Hkv * G, Hkv, int(2 ** rng.uniform(0, 11)), int(2 ** rng.uniform(6, 15)),
+                 rng.choice([64, 128]))
+        kw = dict(dtype=rng.choice(list(DT)), causal=rng.random() < 0.3, fuse_q=rng.choice([-1, 0, 1]))
+        rc, got = run_call(routes, hip_impl, *shape, pv="fp8", **kw)
+        assert rc == 0, got
+        assert got[-1]["nsplit"] == 1, (shape, kw, got)
+        packed += got[-1]["grp"] > 1
+        split += run_call(routes, hip_impl, *shape, pv="fp16", **kw)[1][-1]["nsplit"] > 1
+    assert split > 50 and packed > 5
+
+
+def test_gpu_packed_shapes_pack(routes, hip_impl):
+    """The shapes that test_gpu_attn_split.py means to pack heads with FP8 P do."""
+    from test_gpu_attn_split import PACKED
+
+    for *shape, causal in PACKED:
+        for D in (64, 128):
+            rc, got = run_call(routes, hip_impl, *shape, D, causal=causal, pv="fp8")
+            assert rc == 0 and got[-1]["launch"] == "i8 part" and got[-1]["grp"] > 1, got

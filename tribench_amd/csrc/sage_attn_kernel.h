@@ -1117,7 +1117,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WP
   auto out4 = [&](int dt, int i, TO* p) __attribute__((always_inline)) {
     const int d0 = 32 * dt + 8 * i + 4 * hh;
     float4 f = make_float4(inv, inv, inv, inv);
-    if constexpr (kF8) {
+    if constexpr (kF8 && !kPart) {  // (partial: in the merge, as one factor with 1 / l)
       const float4 vs4 = *reinterpret_cast<const float4*>(vsc + d0);
       f = make_float4(inv * vs4.x, inv * vs4.y, inv * vs4.z, inv * vs4.w);
     }

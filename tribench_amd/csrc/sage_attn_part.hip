@@ -7,7 +7,9 @@
 // grouped KV heads, put the query rows of a group's heads side by side in one
 // work-group; each range's unnormalised O, running max and row sum go to a
 // workspace in fp32, and attn_merge forms
-//   O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s,  M = max_s m_s.
+//   O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s,  M = max_s m_s
+// (times v_scale with FP8 V).  One range (packed heads alone) has weight 1 and
+// the factors of the unsplit kernel's epilogue: its outputs bit for bit.
 #include "sage_attn_kernel.h"
 
 namespace sage {
@@ -59,8 +61,13 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
   if (r0 >= nrow) return;
   const float inv = 1.0f / l;
   const int64_t q = row % a.Nq, bh = row / a.Nq;
+  v4f f = {inv, inv, inv, inv};
+  if (a.v_scale) {  // FP8 V
+    const int64_t hk = bh / a.Hq * a.Hkv + bh % a.Hq / (a.Hq / a.Hkv);
+    f = inv * *reinterpret_cast<const v4f*>(a.v_scale + hk * D + c);
+  }
   TO* p = static_cast<TO*>(a.o) + bh / a.Hq * a.so[0] + bh % a.Hq * a.so[1] + q * a.son + c;
-  store4<TO>(p, o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);
+  store4<TO>(p, o[0] * f[0], o[1] * f[1], o[2] * f[2], o[3] * f[3]);
 }
 
 template <int D, typename TO>
