@@ -39,11 +39,12 @@ typedef struct sage_call {
   int64_t pv_mode;  /* SAGE_PV_* */
   int64_t q_sub;    /* rows per Q scale: 128, 32 or 1 */
   int64_t smooth_k; /* 1: subtract the per-channel K mean */
-  int64_t fuse_q;   /* where Q is quantized: 1 the attention kernel's prologue, 0 the pre-pass, -1 the
-                       faster of the two (the same Q8 and scales, and the same output, bit for bit).
+  int64_t fuse_q;   /* where Q is quantized: 1 the attention kernel's prologue (the pre-pass where the keys
+                       are split or heads share a work-group), 0 the pre-pass, -1 the faster of the two
+                       (the pre-pass with q8): the same Q8 and scales, and the same output, bit for bit.
                        1, and -1 at D = 128, need mul > 0 and finite, a head's Q rows within 2^31 bytes */
   /* optional outputs (NULL: kept in the workspace), as sage_prepass writes them with blkq 128, blkk 64 */
-  void* q8; /* with q's strides when fuse_q is 1, else q8_strides */
+  void* q8; /* with q's strides when fuse_q is 1 (multiples of 16 then), else q8_strides */
   void* q_scale;
   void* k8; /* k8_strides */
   void* k_scale;

@@ -1,0 +1,52 @@
+"""The optional outputs of sage_run in a caller's own layouts.
+
+q is a slice of packed Q, K, V rows and q8 a buffer of its own, at shapes where
+Q is quantized in the attention's prologue, in the pre-pass, and where the keys
+are split or heads share a work-group: Q8 is the pre-pass's bit for bit in the
+layout the options name (q's strides with fuse_q 1, q8_strides otherwise), and
+not a byte beside its rows is written.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from test_run_routes import Q8_SHAPES
+
+pytestmark = pytest.mark.gpu
+CANARY = 77
+
+
+def _strided_q8(shape, strides, dev):
+    """An int8 buffer of canaries and the [B, H, N, D] view of it."""
+    n = sum((a - 1) * b for a, b in zip(shape, strides)) + 1
+    buf = torch.full((n + 256,), CANARY, dtype=torch.int8, device=dev)
+    return buf, buf.as_strided(shape, strides)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("shape", Q8_SHAPES, ids=lambda s: "-".join(map(str, s)))
+def test_q8_layouts(shape, D, hip_impl, gpu_device):
+    B, Hq, Hkv, Nq, Nkv = shape
+    g = torch.Generator().manual_seed(Nq + Nkv)
+    packed = torch.randn(B, Nq, 3, Hq, D, generator=g).to(torch.bfloat16).to(gpu_device)
+    q = packed[:, :, 0].transpose(1, 2)  # rows 3 * Hq * D apart
+    k, v = (torch.randn(B, Hkv, Nkv, D, generator=g).to(torch.bfloat16).to(gpu_device) for _ in range(2))
+    lib = hip_impl._load()
+    mul = float(np.float32(D ** -0.5 * hip_impl.LOG2E_REF))
+    want = hip_impl.prepass(q, k, v)
+    want_o = hip_impl.run(q, k, v)
+    for fuse_q in (-1, 0, 1):
+        print(f"[q8 layout] {shape} D{D} fuse_q {fuse_q}", flush=True)
+        strides = q.stride() if fuse_q == 1 else (Hq * Nq * (D + 16) + 64, Nq * (D + 16), D + 16, 1)
+        buf, q8 = _strided_q8(q.shape, strides, gpu_device)
+        o = torch.empty(q.shape, dtype=q.dtype, device=gpu_device)
+        qs = torch.empty((B, Hq, -(-Nq // 128)), dtype=torch.float32, device=gpu_device)
+        hip_impl.whole_call(lib.sage_run, lib.sage_run_workspace_bytes, "sage_run", q, k, v, o, "HND",
+                            (B, Hq, Hkv, Nq, Nkv, D), mul, False, 0, 128, 1, fuse_q, [q8, qs, None, None, None, None])
+        torch.cuda.synchronize()
+        assert torch.equal(q8, want["q8"]) and torch.equal(qs, want["q_scale"])
+        assert torch.equal(o, want_o)
+        q8.fill_(CANARY)
+        assert (buf == CANARY).all()

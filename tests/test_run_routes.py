@@ -21,6 +21,7 @@ BUF, Q8 = 1 << 20, 1 << 21  # addresses nothing reads
 
 @pytest.fixture(scope="module")
 def routes(tmp_path_factory, hip_impl):
+    hip_impl._load()  # (first: as a dependency of the stand-ins it would bind to them)
     so = hip_impl.library_path()
     out = tmp_path_factory.mktemp("routes") / "run_routes.so"
     subprocess.run([hip_build.hipcc(), *hip_build.COMMON, "-O0", "-w", "-shared", "-x", "hip",
@@ -86,3 +87,44 @@ def test_gpu_packed_shapes_pack(routes, hip_impl):
         for D in (64, 128):
             rc, got = run_call(routes, hip_impl, *shape, D, causal=causal, pv="fp8")
             assert rc == 0 and got[-1]["launch"] == "i8 part" and got[-1]["grp"] > 1, got
+
+
+# (B, Hq, Hkv, Nq, Nkv): Q in the prologue when left to choose; two that split the keys; packed heads
+Q8_SHAPES = [(4, 32, 8, 512, 512), (1, 4, 2, 300, 4096), (2, 8, 2, 5, 3000), (64, 32, 8, 1, 200)]
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("shape", Q8_SHAPES, ids=lambda s: "-".join(map(str, s)))
+def test_q8_layout_follows_the_options(routes, hip_impl, shape, D):
+    """A caller's q8 has q's strides with fuse_q 1 and q8_strides otherwise,
+    whatever launches the shape takes; q is a slice of packed Q, K, V rows."""
+    B, Hq, Hkv, Nq, Nkv = shape
+    q_strides = [Nq * 3 * Hq * D, D, 3 * Hq * D]
+    q8_strides = [Hq * Nq * D + 64, Nq * D, D]
+    outs = [Q8, BUF, 0, 0, 0, 0]
+    seen = set()
+    for fuse_q in (-1, 0, 1):
+        # (with fuse_q 1 the caller need not fill q8_strides)
+        rc, got = run_call(routes, hip_impl, *shape, D, fuse_q=fuse_q, q_strides=q_strides, outs=outs,
+                           q8_strides=None if fuse_q == 1 else q8_strides)
+        assert rc == 0, got
+        pre, attn = got
+        want = q_strides if fuse_q == 1 else q8_strides
+        if pre["quant_q"]:
+            assert pre["q8"] == Q8 and pre["q8_strides"] == want and attn["q_strides"] == want, got
+        else:
+            assert attn["q8_out"] == Q8 and attn["q_strides"] == q_strides == want, got
+        seen.add(attn["launch"])
+    assert ("i8 part" in seen) == (shape != Q8_SHAPES[0]), seen
+
+
+def test_q8_rows_stay_aligned(routes, hip_impl):
+    """q8 with q's strides is refused by those strides, not by the launch."""
+    for shape in Q8_SHAPES:
+        D = 64
+        q_strides = [shape[1] * shape[3] * 72, shape[3] * 72, 72]
+        kw = dict(q_strides=q_strides, outs=[Q8, BUF, 0, 0, 0, 0])
+        rc, msg = run_call(routes, hip_impl, *shape, D, fuse_q=1, **kw)
+        assert rc != 0 and "invalid argument" in msg and "q8" in msg, msg
+        for fuse_q in (-1, 0):
+            assert run_call(routes, hip_impl, *shape, D, fuse_q=fuse_q, q8_strides=dense(shape[1], shape[3], D), **kw)[0] == 0

@@ -412,8 +412,9 @@ static RunPlan run_plan(const sage_call* c) {
   // faster per call (226 keys, B2 H48 N17776 D64: 267 us against 292), with
   // fewer the start is what counts and the pre-pass is 1 to 9 % faster (B1 H18
   // N159 D128: 24.6 us against 26.8).
-  // (the prologue takes only what sage_attn_fwd_q does: q_fusable)
-  r.fuse_q = c->fuse_q < 0 ? (c->Nq + 127) / 128 * c->Hq * c->B > 256 && q_fusable(*c) : c->fuse_q != 0;
+  // (the prologue takes only what sage_attn_fwd_q does: q_fusable; it writes a
+  // caller's Q8 with q's strides, which is the layout of fuse_q 1 alone)
+  r.fuse_q = c->fuse_q < 0 ? (c->Nq + 127) / 128 * c->Hq * c->B > 256 && q_fusable(*c) && !c->q8 : c->fuse_q != 0;
   r.quant_q = !r.fuse_q || r.attn.part();  // the partial kernels read Q8
   // V already in the P.V type: read in place, no V tiles (4 bytes of traffic
   // per element less: fp16 B8 H16 N4096 D64 548 us -> 536, 32 rows over 16384
@@ -471,7 +472,9 @@ extern "C" int sage_run(const sage_call* c, void* stream) {
 
   const int64_t q8_dense[3] = {c->Hq * c->Nq * c->D, c->Nq * c->D, c->D};
   const int64_t k8_dense[3] = {c->Hkv * c->Nkv * c->D, c->Nkv * c->D, c->D};
-  const int64_t* q8_strides = c->q8 ? c->q8_strides : q8_dense;
+  // the layout of a caller's Q8 goes by the options, not by which launch writes it
+  const bool q8_as_q = c->q8 && c->fuse_q > 0;
+  const int64_t* q8_strides = q8_as_q ? c->q_strides : c->q8 ? c->q8_strides : q8_dense;
   const int64_t* k8_strides = c->k8 ? c->k8_strides : k8_dense;
   int8_t* q8 = static_cast<int8_t*>(c->q8 || !r.quant_q ? c->q8 : ws + r.off_q8);
   float* qs = static_cast<float*>(c->q_scale || !r.quant_q ? c->q_scale : ws + r.off_qs);
@@ -486,6 +489,8 @@ extern "C" int sage_run(const sage_call* c, void* stream) {
     if (!(mul > 0.0f) || mul == INFINITY) return fail("%s: invalid argument: mul %g", who, mul);
     return fail("%s: invalid argument: a head's rows must span < 2^31 bytes", who);
   }
+  if (q8_as_q && !strides_ok(c->q_strides, 1))
+    return fail("%s: invalid argument: q8 with q's strides must keep 16-byte aligned rows", who);
 
   const int pv = (int)c->pv_mode, dt = (int)c->dtype, q_sub = (int)c->q_sub;
   const bool dq = r.quant_q;
