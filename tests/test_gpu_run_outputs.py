@@ -4,7 +4,8 @@ q is a slice of packed Q, K, V rows and q8 a buffer of its own, at shapes where
 Q is quantized in the attention's prologue, in the pre-pass, and where the keys
 are split or heads share a work-group: Q8 is the pre-pass's bit for bit in the
 layout the options name (q's strides with fuse_q 1, q8_strides otherwise), and
-not a byte beside its rows is written.
+not a byte beside its rows is written.  A call whose outputs are all the
+caller's and that needs no other buffer runs without a workspace.
 """
 from __future__ import annotations
 
@@ -50,3 +51,23 @@ def test_q8_layouts(shape, D, hip_impl, gpu_device):
         assert torch.equal(o, want_o)
         q8.fill_(CANARY)
         assert (buf == CANARY).all()
+
+
+@pytest.mark.parametrize("fuse_q", [None, True, False])
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", [(4, 32, 32, 640, 128), (1, 2, 2, 256, 64), (16, 48, 12, 193, 64)],
+                         ids=lambda s: "-".join(map(str, s)))
+def test_intermediates_without_smoothing(shape, dtype, fuse_q, hip_impl, gpu_device):
+    print(f"[no smoothing] {shape} {dtype} fuse_q {fuse_q}", flush=True)
+    B, Hq, Hkv, N, D = shape
+    dt = torch.float16 if dtype == "fp16" else torch.bfloat16
+    g = torch.Generator().manual_seed(N)
+    q, k, v = (torch.randn(B, h, N, D, generator=g).to(dt).to(gpu_device) for h in (Hq, Hkv, Hkv))
+    o, pre = hip_impl.run(q, k, v, pv_dtype=dtype, smooth_k=False, fuse_q=fuse_q, return_intermediates=True)
+    want = hip_impl.prepass(q, k, v, smooth_k=False)
+    torch.cuda.synchronize()
+    assert sorted(pre) == ["k8", "k_scale", "q8", "q_scale"]
+    for key in pre:
+        assert torch.equal(pre[key], want[key]), key
+    assert torch.equal(o, hip_impl.run(q, k, v, pv_dtype=dtype, smooth_k=False))
+    assert torch.equal(o, hip_impl.attention(q, k, v, want, pv_dtype=dtype))

@@ -128,3 +128,20 @@ def test_q8_rows_stay_aligned(routes, hip_impl):
         assert rc != 0 and "invalid argument" in msg and "q8" in msg, msg
         for fuse_q in (-1, 0):
             assert run_call(routes, hip_impl, *shape, D, fuse_q=fuse_q, q8_strides=dense(shape[1], shape[3], D), **kw)[0] == 0
+
+
+@pytest.mark.parametrize("fuse_q", [0, 1])
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", [(4, 32, 32, 1024, 1024, 128), (1, 2, 2, 256, 256, 64)],
+                         ids=lambda s: "-".join(map(str, s)))
+def test_no_workspace_needed(routes, hip_impl, shape, dtype, fuse_q):
+    """Every output given, no K smoothing, V in place and one sweep: nothing to
+    keep in a workspace, and the call runs without one."""
+    B, Hq, Hkv, Nq, Nkv, D = shape
+    kw = dict(dtype=dtype, pv=dtype, fuse_q=fuse_q, smooth_k=0, outs=[BUF] * 4 + [0, 0], q8_strides=dense(Hq, Nq, D),
+              k8_strides=dense(Hkv, Nkv, D))
+    rc, got = run_call(routes, hip_impl, *shape, **kw)
+    assert rc == 0, got
+    pre, attn = got
+    assert attn["vrow"] == 1 and attn["nsplit"] == 1 and pre["quant_q"] == 1 - fuse_q
+    assert run_call(routes, hip_impl, *shape, **{**kw, "smooth_k": 1})[0] == 0  # (a workspace for the sums)

@@ -467,7 +467,7 @@ extern "C" int sage_run(const sage_call* c, void* stream) {
   if (!run_options_ok(c)) return fail("%s: invalid argument: q_sub or pv_mode", who);
   const RunPlan r = run_plan(c);
   char* ws = static_cast<char*>(c->workspace);
-  if (!ws || (size_t)c->workspace_bytes < r.bytes || (uintptr_t)ws % 256 != 0)
+  if (r.bytes && (!ws || (size_t)c->workspace_bytes < r.bytes || (uintptr_t)ws % 256 != 0))
     return fail("%s: invalid argument: workspace (%zu bytes, 256-byte aligned)", who, r.bytes);
 
   const int64_t q8_dense[3] = {c->Hq * c->Nq * c->D, c->Nq * c->D, c->D};
