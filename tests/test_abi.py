@@ -261,3 +261,21 @@ def test_sage_run_limits_do_not_depend_on_the_shape(lib, hip_impl, Hq):
         assert lib.sage_run(_sage_call(hip_impl, Hq=Hq, **over), None) != 0  # no device: the launch fails
         msg = lib.sage_last_error().decode()
         assert "invalid argument" not in msg, msg
+
+
+@pytest.mark.parametrize("pack", ["sage_attn", "flash_attn"])
+def test_packs_load_on_a_torch_without_a_gpu_backend(pack, hip_impl, monkeypatch):
+    """Such a build has no raw stream query; the packs load and the call names
+    the missing device."""
+    import importlib.util
+
+    import torch
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    path = ROOT / "tribench_amd" / "kernels" / pack / "hip_impl.py"
+    spec = importlib.util.spec_from_file_location(f"no_backend_{pack}", path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    q = torch.zeros(1, 2, 16, 64, dtype=torch.float16)
+    with pytest.raises(RuntimeError, match="ROCm GPU device"):
+        mod.run(q, q, q)

@@ -158,8 +158,10 @@ def _stream(device) -> ctypes.c_void_p:
 _CALL = struct.Struct("@q6P18q1d6q6P6q")  # sage_call (include/sage_attn_run.h)
 _CALL_SIZE = _CALL.size
 _CALL_WS = struct.Struct("@2q")
-_raw_stream = torch._C._cuda_getCurrentRawStream  # the handle alone: no Stream object per call
 _CALL_WS_AT = 40  # byte offset of its workspace fields
+# the handle alone, no Stream object per call (a torch without a GPU backend lacks the query)
+_raw_stream = (getattr(torch._C, "_cuda_getCurrentRawStream", None)
+               or (lambda index: torch.cuda.current_stream(index).cuda_stream))
 
 
 def whole_call(fn, fn_bytes, what, q, k, v, o, layout, dims, mul, causal, pv_mode=0, q_sub=0, smooth_k=0, fuse_q=0, outs=None):
