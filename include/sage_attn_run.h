@@ -57,6 +57,10 @@ typedef struct sage_call {
 size_t sage_run_workspace_bytes(const sage_call* call);
 size_t sage_flash_run_workspace_bytes(const sage_call* call);
 
+/* Which parts of the pre-pass sage_run() makes for this call: Q quantized there (or in the attention's
+   prologue), V tiles (or V read in place).  For whoever times or repeats the stages one by one. */
+int sage_run_stages(const sage_call* call, int* quant_q, int* v_tiles);
+
 /* SageAttention forward: sage_prepass_vt and the fused attention. */
 int sage_run(const sage_call* call, void* stream);
 

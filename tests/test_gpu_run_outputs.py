@@ -71,3 +71,25 @@ def test_intermediates_without_smoothing(shape, dtype, fuse_q, hip_impl, gpu_dev
         assert torch.equal(pre[key], want[key]), key
     assert torch.equal(o, hip_impl.run(q, k, v, pv_dtype=dtype, smooth_k=False))
     assert torch.equal(o, hip_impl.attention(q, k, v, want, pv_dtype=dtype))
+
+
+# (B, Hq, Hkv, Nq, Nkv, D), dtype, pv, whether the pre-pass of the call has Q and V tiles
+STAGES = [((1, 32, 32, 1100, 1100, 128), "bf16", "fp16", False, True),
+          ((2, 24, 24, 900, 900, 64), "fp16", "fp16", False, False),
+          ((1, 2, 2, 256, 256, 64), "bf16", "fp8", True, True),
+          ((2, 8, 2, 32, 3000, 128), "bf16", "bf16", True, False)]
+
+
+@pytest.mark.parametrize("case", STAGES, ids=lambda c: "-".join(map(str, c[0])))
+def test_prepass_stage_is_runs(case, hip_impl, gpu_device):
+    """The timed stage makes what run's own pre-pass makes, no more and no less."""
+    (B, Hq, Hkv, Nq, Nkv, D), dtype, pv, has_q, has_vt = case
+    dt = torch.float16 if dtype == "fp16" else torch.bfloat16
+    g = torch.Generator().manual_seed(Nkv)
+    q, k, v = (torch.randn(B, h, n, D, generator=g).to(dt).to(gpu_device) for h, n in ((Hq, Nq), (Hkv, Nkv), (Hkv, Nkv)))
+    pre = hip_impl.prepass_stage(q, k, v, pv_dtype=pv)
+    _, want = hip_impl.run(q, k, v, pv_dtype=pv, return_intermediates=True, fuse_q=False)
+    torch.cuda.synchronize()
+    assert ("q8" in pre, "vt" in pre) == (has_q, has_vt)
+    for key in set(pre) & set(want):
+        assert torch.equal(pre[key], want[key]), key

@@ -236,6 +236,19 @@ def test_estimate(pack_ref):
     assert c["flops"] == 2 ** 43 and c["algo_flops"] == O.attention_flops(2, 32, 16384, 16384, 128, True)[1]
 
 
+def test_prepass_bytes_follow_the_stage(pack_ref):
+    """The pre-pass's rate counts what the stage did: Q and V only if it wrote them."""
+    from tribench_amd.harness.bench import prepass_bytes
+
+    e = pack_ref.estimate(dict(batch_size=4, num_heads=32, seq_len=4096, head_dim=128))
+    kn = 4 * 32 * 4096 * 128
+    k_only = 3 * kn + 4 * 4 * 32 * 64 + 4 * 4 * 32 * 128
+    assert prepass_bytes(e, {"k8": 0}) == k_only
+    assert prepass_bytes(e, {"k8": 0, "q8": 0}) == k_only + 3 * kn + 4 * 4 * 32 * 32
+    assert prepass_bytes(e, {"k8": 0, "vt": 0}) == k_only + 4 * kn
+    assert prepass_bytes({}, {"k8": 0}) is None
+
+
 # ---------------------------------------------------------------------------
 # correctness gate / metrics
 # ---------------------------------------------------------------------------

@@ -52,12 +52,18 @@ def run_call(lib, hip_impl, B, Hq, Hkv, Nq, Nkv, D, *, flash=False, dtype="bf16"
                                    B, Hq, Hkv, Nq, Nkv, D, 0.1, DT[dtype], int(causal), PV[pv], q_sub, smooth_k,
                                    fuse_q, *(outs or [0] * 6), *(q8_strides or [0] * 3), *(k8_strides or [0] * 3))
 
+    if not flash:
+        quant_q, v_tiles = ctypes.c_int(-1), ctypes.c_int(-1)
+        assert lib.sage_run_stages(pack(0, 0), ctypes.byref(quant_q), ctypes.byref(v_tiles)) == 0
     n = getattr(lib, name + "_workspace_bytes")(pack(0, 0))
     lib.take_routes()
     rc = getattr(lib, name)(pack(BUF if n else 0, n), None)
     if rc:
         return rc, lib.sage_last_error().decode()
-    return 0, [json.loads(line) for line in lib.take_routes().decode().splitlines()]
+    got = [json.loads(line) for line in lib.take_routes().decode().splitlines()]
+    if not flash:  # sage_run_stages says what the call then does
+        assert (quant_q.value, v_tiles.value) == (got[0]["quant_q"], got[0]["v"]) == (got[0]["quant_q"], 1 - got[1]["vrow"])
+    return 0, got
 
 
 def test_fp8_keys_stay_in_one_sweep(routes, hip_impl):
@@ -145,3 +151,18 @@ def test_no_workspace_needed(routes, hip_impl, shape, dtype, fuse_q):
     pre, attn = got
     assert attn["vrow"] == 1 and attn["nsplit"] == 1 and pre["quant_q"] == 1 - fuse_q
     assert run_call(routes, hip_impl, *shape, **{**kw, "smooth_k": 1})[0] == 0  # (a workspace for the sums)
+
+
+def test_stages_of_typical_calls(routes, hip_impl):
+    """What the harness times as run's pre-pass: Q where few blocks or a split
+    want it there, V tiles where V is not of the P.V type."""
+    for shape, kw, quant_q, v in [
+        ((4, 32, 32, 4096, 4096, 128), dict(dtype="bf16"), 0, 1),
+        ((8, 16, 16, 4096, 4096, 64), dict(dtype="fp16"), 0, 0),
+        ((1, 2, 2, 256, 256, 64), dict(dtype="bf16"), 1, 1),
+        ((2, 32, 8, 32, 16384, 128), dict(dtype="fp16"), 1, 0),
+        ((2, 32, 8, 32, 16384, 128), dict(dtype="fp16", fuse_q=1), 1, 0),  # split: Q8 comes from the pre-pass
+        ((1, 8, 8, 512, 512, 128), dict(dtype="bf16", pv="fp8", fuse_q=1), 0, 1),
+    ]:
+        rc, got = run_call(routes, hip_impl, *shape, **kw)
+        assert rc == 0 and (got[0]["quant_q"], got[0]["v"]) == (quant_q, v), (shape, kw, got)

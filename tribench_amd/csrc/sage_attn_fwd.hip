@@ -458,13 +458,28 @@ extern "C" size_t sage_run_workspace_bytes(const sage_call* c) {
   return run_plan(c).bytes;
 }
 
-extern "C" int sage_run(const sage_call* c, void* stream) {
-  const char* who = "sage_run";
+static int run_check(const char* who, const sage_call* c) {
   if (!call_ok(c)) return fail("%s: invalid argument: sage_call size", who);
   if (!shape_ok(c)) return fail("%s: invalid argument: empty shape or Hq %% Hkv != 0", who);
   if (c->D != 64 && c->D != 128)
     return fail("%s: invalid argument: head_dim %lld (supported: 64, 128)", who, (long long)c->D);
   if (!run_options_ok(c)) return fail("%s: invalid argument: q_sub or pv_mode", who);
+  return 0;
+}
+
+extern "C" int sage_run_stages(const sage_call* c, int* quant_q, int* v_tiles) {
+  const char* who = "sage_run_stages";
+  if (int rc = run_check(who, c)) return rc;
+  if (!quant_q || !v_tiles) return fail("%s: invalid argument: null pointer", who);
+  const RunPlan r = run_plan(c);
+  *quant_q = r.quant_q;
+  *v_tiles = !r.vrow;
+  return 0;
+}
+
+extern "C" int sage_run(const sage_call* c, void* stream) {
+  const char* who = "sage_run";
+  if (int rc = run_check(who, c)) return rc;
   const RunPlan r = run_plan(c);
   char* ws = static_cast<char*>(c->workspace);
   if (r.bytes && (!ws || (size_t)c->workspace_bytes < r.bytes || (uintptr_t)ws % 256 != 0))

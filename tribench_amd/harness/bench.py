@@ -185,15 +185,23 @@ def run_benchmark(
     res.roofline_fraction = (rate / peak) if (rate and peak) else None
     pre_fn = (stage_fns or {}).get("prepass")
     if pre_fn is not None and device.startswith("cuda"):
+        pb = prepass_bytes(est, pre_fn(**inputs))
         pre_p50 = stats.summarize(timer(lambda: pre_fn(**inputs), warmup_ms / 4, rep_ms / 4)).p50
         res.prepass_ms_p50 = pre_p50
-        pb = est.get("prepass_bytes")
-        if pb and est.get("vtile_bytes"):
-            pb += est["vtile_bytes"]  # the stage also converts V (v.to(float16))
         if pb:
             res.prepass_gbps = compute_gbps(pb, pre_p50)
             res.prepass_hbm_fraction = res.prepass_gbps / PEAKS_MI355X["hbm_gbps"]
     return res
+
+
+def prepass_bytes(est: dict, outputs: dict) -> float | None:
+    """Algorithmic bytes of a ``prepass`` stage by what it wrote: without Q
+    where the attention quantizes it, the conversion of V to the P.V type
+    (v.to(float16)) where it made V tiles."""
+    pb = est.get("prepass_bytes" if "q8" in outputs else "prepass_bytes_k")
+    if pb and "vt" in outputs:
+        pb += est.get("vtile_bytes", 0)
+    return pb
 
 
 def run_cpu_reference(

@@ -117,6 +117,8 @@ def _load():
         getattr(lib, name).argtypes = [ctypes.c_char_p, vp]
         getattr(lib, name + "_workspace_bytes").restype = sz
         getattr(lib, name + "_workspace_bytes").argtypes = [ctypes.c_char_p]
+    lib.sage_run_stages.restype = i32
+    lib.sage_run_stages.argtypes = [ctypes.c_char_p, ctypes.POINTER(i32), ctypes.POINTER(i32)]
     _LIB = lib
     return lib
 
@@ -370,7 +372,7 @@ def q_sub_of(q_gran):
 
 
 def fuse_q_default(head_dim):
-    """Where the stage calls (and intermediates) have Q quantized when the caller
+    """Where stage calls (and run's intermediates) have Q quantized when the caller
     does not say: in the attention kernel's prologue at D = 128 (measured 1-2 % faster per forward at
     configurations 2 and 3, even at 5), in the pre-pass at D = 64 (the
     prologue costs more than it saves there: 2 % slower at configuration 4)."""
@@ -381,12 +383,19 @@ def fuse_q_default(head_dim):
 def prepass_stage(q, k, v, causal=False, sm_scale=None, *, pv_dtype="fp16", q_gran="block", smooth_k=True,
                   fuse_q=None, tensor_layout="HND", **kw):
     """The pre-pass of :func:`run` alone, with run's arguments (the harness
-    times it as the ``prepass`` stage to report its HBM rate)."""
+    times it as the ``prepass`` stage to report its HBM rate): what run leaves
+    to the attention (Q in its prologue, V read in place) is left out."""
+    if pv_dtype not in PV_MODES:
+        raise ValueError(f"sage_attn hip: invalid argument: pv_dtype {pv_dtype!r}")
     q_sub = q_sub_of(q_gran)
-    if fuse_q is None:
-        fuse_q = fuse_q_default(_dims(q, tensor_layout)[3])
-    return prepass(q, k, v, sm_scale, q_sub=q_sub, smooth_k=smooth_k, pv_dtype=pv_dtype, quant_q=not fuse_q,
-                   tensor_layout=tensor_layout)
+    dims = _check_inputs(q, k, v, tensor_layout)
+    lib, quant_q, v_tiles = _load(), ctypes.c_int(), ctypes.c_int()
+    mul = float(np.float32((dims[5] ** -0.5 if sm_scale is None else sm_scale) * LOG2E_REF))
+    whole_call(lambda call, _: lib.sage_run_stages(call, quant_q, v_tiles), lambda _: 0, "sage_run_stages", q, k, v, q,
+               tensor_layout, dims, mul, causal, PV_MODES[pv_dtype], q_sub, int(bool(smooth_k)),
+               -1 if fuse_q is None else int(bool(fuse_q)))
+    return prepass(q, k, v, sm_scale, q_sub=q_sub, smooth_k=smooth_k, pv_dtype=pv_dtype if v_tiles.value else None,
+                   quant_q=bool(quant_q.value), tensor_layout=tensor_layout)
 
 
 @_on_tensor_device
