@@ -48,7 +48,7 @@
 extern "C" {
 #endif
 
-#define SAGE_ABI_VERSION 6
+#define SAGE_ABI_VERSION 7
 
 /* element types (dtype codes used by every entry point) */
 #define SAGE_DTYPE_F32 0
@@ -68,7 +68,7 @@ extern "C" {
 #define SAGE_PV_BF16 1 /* P and V in bf16 */
 #define SAGE_PV_FP8 2  /* P and V in FP8 e4m3 with per-channel V scales */
 
-/* Library version; bumped whenever a signature below changes. */
+/* Library version; bumped whenever a signature here or in sage_attn_run.h changes or is added. */
 int sage_abi_version(void);
 
 /* Message of the last failed call on the calling thread ("" if none). */

@@ -1,19 +1,22 @@
 """The C-ABI library on a host without a GPU: it loads, exports every symbol
-of include/sage_attn.h, and rejects bad arguments before touching a device."""
+of include/sage_attn.h and sage_attn_run.h, and rejects bad arguments before
+touching a device."""
 from __future__ import annotations
 
 import ctypes
 import re
+import subprocess
 from pathlib import Path
 
 import pytest
 
 ROOT = Path(__file__).resolve().parents[1]
 HEADER = ROOT / "include" / "sage_attn.h"
+RUN_HEADER = ROOT / "include" / "sage_attn_run.h"
 
 
-def _declared_functions():
-    text = HEADER.read_text()
+def _declared_functions(header=HEADER):
+    text = header.read_text()
     text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
     return sorted(set(re.findall(r"\b(sage_[a-z_0-9]+)\s*\(", text)))
 
@@ -30,9 +33,9 @@ def test_header_declares_the_entry_points():
                                      "sage_vtile_bytes", "sage_vtiles"]
 
 
-def _declared_arg_counts():
+def _declared_arg_counts(header=HEADER):
     """Parameter count of every function declared in the header."""
-    text = re.sub(r"/\*.*?\*/", "", HEADER.read_text(), flags=re.S)
+    text = re.sub(r"/\*.*?\*/", "", header.read_text(), flags=re.S)
     out = {}
     for name, params in re.findall(r"\b(sage_[a-z_0-9]+)\s*\(([^;{]*?)\)\s*;", text, flags=re.S):
         params = params.strip()
@@ -279,3 +282,56 @@ def test_packs_load_on_a_torch_without_a_gpu_backend(pack, hip_impl, monkeypatch
     q = torch.zeros(1, 2, 16, 64, dtype=torch.float16)
     with pytest.raises(RuntimeError, match="ROCm GPU device"):
         mod.run(q, q, q)
+
+
+def test_run_header_declares_what_the_binding_calls(lib):
+    counts = _declared_arg_counts(RUN_HEADER)
+    assert sorted(counts) == _declared_functions(RUN_HEADER) == [
+        "sage_flash_run", "sage_flash_run_workspace_bytes", "sage_run", "sage_run_stages", "sage_run_workspace_bytes"]
+    for name, n in counts.items():
+        assert len(getattr(lib, name).argtypes) == n, name
+
+
+def test_sage_call_layout_matches_the_header(hip_impl, tmp_path):
+    """The binding packs sage_call field by field where the C compiler puts them."""
+    text = re.sub(r"/\*.*?\*/", "", RUN_HEADER.read_text(), flags=re.S)
+    body = re.search(r"typedef struct sage_call \{(.*?)\} sage_call;", text, flags=re.S).group(1)
+    fields = []  # (name, struct code, count)
+    for ctype, names in re.findall(r"(const void\s*\*|void\s*\*|int64_t|double)\s*([^;]+);", body):
+        for name in names.split(","):
+            m = re.fullmatch(r"\s*(\w+)(?:\[(\d+)\])?\s*", name)
+            fields.append((m.group(1), "P" if "*" in ctype else {"int64_t": "q", "double": "d"}[ctype],
+                           int(m.group(2) or 1)))
+    assert "".join(code * n for _, code, n in fields) == "".join(
+        code * int(n or 1) for n, code in re.findall(r"(\d*)([qPd])", hip_impl._CALL.format))
+    src = tmp_path / "layout.c"
+    src.write_text('#include <stddef.h>\n#include <stdio.h>\n#include "sage_attn_run.h"\nint main(void) {\n'
+                   + "".join(f'  printf("%zu\\n", offsetof(sage_call, {name}));\n' for name, _, _ in fields)
+                   + '  printf("%zu\\n", sizeof(sage_call));\n  return 0;\n}\n')
+    exe = tmp_path / "layout"
+    subprocess.run(["gcc", f"-I{RUN_HEADER.parent}", "-o", str(exe), str(src)], check=True)
+    got = [int(x) for x in subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split()]
+    want, at = [], 0
+    for _, _, n in fields:
+        want.append(at)
+        at += 8 * n
+    assert got == want + [hip_impl._CALL_SIZE]
+    assert dict(zip((f[0] for f in fields), got))["workspace"] == hip_impl._CALL_WS_AT
+
+
+def test_a_library_without_the_whole_call_is_refused_by_version(monkeypatch, tmp_path):
+    """A library of the ABI before sage_attn_run.h is told to rebuild, not
+    tripped over by its missing symbols."""
+    import importlib.util
+
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text("int sage_abi_version(void) { return 6; }\n"
+                   + "".join(f"void {n}(void) {{}}\n" for n in _declared_functions() if n != "sage_abi_version"))
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    monkeypatch.setenv("TRIBENCH_SAGE_HIP_LIB", str(so))
+    spec = importlib.util.spec_from_file_location("old_lib_impl", ROOT / "tribench_amd" / "kernels" / "sage_attn" /
+                                                  "hip_impl.py")
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    with pytest.raises(RuntimeError, match="ABI 6.*rebuild"):
+        mod._load()

@@ -31,7 +31,7 @@ from pathlib import Path
 import numpy as np
 import torch
 
-ABI_VERSION = 6
+ABI_VERSION = 7
 LOG2E_REF = 1.44269504  # triton_impl.py:69
 WAVE_ROWS = 32          # q rows per wavefront of the attention kernel (q_gran="wave")
 # rows per Q scale for each q_gran: one block of 128 rows (the reference), one
@@ -157,7 +157,7 @@ def _stream(device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
-_CALL = struct.Struct("@q6P18q1d6q6P6q")  # sage_call (include/sage_attn_run.h)
+_CALL = struct.Struct("@q5P19q1d6q6P6q")  # sage_call (include/sage_attn_run.h)
 _CALL_SIZE = _CALL.size
 _CALL_WS = struct.Struct("@2q")
 _CALL_WS_AT = 40  # byte offset of its workspace fields
