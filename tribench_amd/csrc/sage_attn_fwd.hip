@@ -67,8 +67,7 @@ static AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_
     }
   };
   consider(1, 1);
-  // (FP8 P with fp32 outputs spills there: 685 us -> 794 at B4 H48 N3801)
-  if (D == 64 && !(i8 && pv_mode == SAGE_PV_FP8 && dtype == SAGE_DTYPE_F32)) {
+  if (D == 64 && wpe3_fits(i8, pv_mode, dtype == SAGE_DTYPE_F32)) {
     // Three 4-wave work-groups to a CU hide more of each one's start, without
     // the second S buffer (168 VGPRs): a block takes 1.5x (INT8) to 1.7x as
     // long, shared by three.  226 keys: 267 us -> 215 per call (B2 H48

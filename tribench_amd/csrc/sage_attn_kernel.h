@@ -1211,9 +1211,13 @@ int launch_attn_wpe(const AttnArgs& a, hipStream_t st, const char* who) {
   return check_launch(who);
 }
 
+// FP8 P with fp32 outputs does not fit the registers of three waves per SIMD
+// (685 us -> 794 at B4 H48 N3801), so that kernel is not built or chosen.
+constexpr bool wpe3_fits(bool i8, int pv_mode, bool o_f32) { return !(i8 && pv_mode == SAGE_PV_FP8 && o_f32); }
+
 template <int QKM, int D, int PVM, typename TO, int NW, bool kVRow>
 int launch_attn_nw(const AttnArgs& a, hipStream_t st, const char* who) {
-  if constexpr (D == 64 && NW == 4)
+  if constexpr (D == 64 && NW == 4 && wpe3_fits(QKM == kQkI8 || QKM == kQkI8Q, PVM, std::is_same_v<TO, float>))
     if (a.wpe == 3) return launch_attn_wpe<QKM, D, PVM, TO, NW, 3, kVRow>(a, st, who);
   return launch_attn_wpe<QKM, D, PVM, TO, NW, 2, kVRow>(a, st, who);
 }
