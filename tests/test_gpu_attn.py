@@ -68,14 +68,14 @@ SMALL = [
     (2, 4, 2, 300, 128, "bf16", True, "fp16", "thread", 2.0),  # per-row Q scales
     (1, 3, 3, 1000, 64, "fp16", False, "fp16", "thread", 4.0),
     (1, 2, 2, 777, 128, "bf16", True, "fp16", "thread", 2.0),
-    # non-causal N = 64 * nkb runs nkb - 4 mask-free iterations (blocks 1 ..
-    # nkb - 4), in trips of 2 at D = 128 and of 10, then 5, at D = 64, then
-    # one at a time: these end the trips with and without leftovers
+    # non-causal sweeps of nkb whole blocks run nkb - 4 mask-free iterations, in
+    # trips of 2 at D = 128 and of 4 at D = 64 (every leftover, in every kernel:
+    # test_gpu_launches.py); the last two are split over the keys
     (1, 2, 2, 448, 128, "bf16", False, "fp16", "block", 2.0),   # 3 = one 2-trip + 1
     (1, 2, 2, 512, 128, "bf16", False, "fp16", "wave", 2.0),    # 4 = two 2-trips
-    (1, 2, 1, 896, 64, "bf16", False, "fp16", "block", 2.0),    # 10 = one 10-trip
-    (1, 2, 2, 1216, 64, "fp16", False, "fp16", "block", 2.0),   # 15 = 10 + 5
-    (1, 1, 1, 1408, 64, "bf16", False, "fp16", "thread", 2.0),  # 18 = 10 + 5 + 3
+    (1, 2, 1, 896, 64, "bf16", False, "fp16", "block", 2.0),    # 10 = two 4-trips + 2
+    (1, 2, 2, 1216, 64, "fp16", False, "fp16", "block", 2.0),   # 8 ranges of 3 blocks, one short, one empty
+    (1, 1, 1, 1408, 64, "bf16", False, "fp16", "thread", 2.0),  # 12 ranges of 2, the last empty
     # bf16 P with fp16 outputs, on short and causal rows (P's rounding shows)
     (1, 6, 2, 178, 64, "fp16", False, "bf16", "wave", 2.0),
     (2, 2, 1, 1318, 128, "fp16", True, "bf16", "block", 2.0),
@@ -249,7 +249,9 @@ def rising_inputs(B, H, N, D, step, seed):
 # blocks move a row's running max by more than the lazy-rescale threshold of
 # 8, a third by more than 7).  In the mask-free loop the shortcut that forms P
 # against the running max then fails its bound and the block is redone, and
-# lazy O rescales happen throughout.  The keys' large values cost INT8
+# lazy O rescales happen throughout.  (These shapes are split over the keys, so
+# ranges with maxima far apart meet in the merge; unsplit sweeps with rising
+# scores are in test_gpu_launches.py.)  The keys' large values cost INT8
 # accuracy (the emulation itself is up to 4.7e-2 off SDPA here), so the
 # kernel is held to the emulation bound and SDPA to the cosine only.
 # (B, H, N, D, dtype, causal, pv, q_gran)

@@ -3,12 +3,15 @@
 ``run`` chooses the split and the packing of grouped heads by the shape; the
 stage entry points (``attention`` on the pre-pass's own outputs, sage_flash_fwd
 on V tiles) always sweep all keys at once.  Q8, K8 and the scales are the same;
-P is rounded to its type against another running max (e_p = 2^-11 fp16, 2^-9
-bf16, relative), the row sums of fp16 P carry 5 * 2^-11 each, and O is rounded
-to its type (e_o), so
+P is rounded to its type against another running max (e_p, relative: half an
+ulp, 2^-11 fp16, 2^-8 bf16 with its 8 significant bits), the row sums of fp16 P
+carry 5 * 2^-11 each, and O is rounded to its type (e_o), so
   |a - b| <= 2 e_p max|v| + (2 e_o + 10 * 2^-11) |o|.
+The roundings of P are independent of V, so the relative 2-norm of a - b is
+within their rms on both sides, 2 e_p / sqrt(3), plus 2 e_o + 10 * 2^-11.
 FP8 P would move by 2^-4, the type's whole error, so its keys are not split; its
-packed heads sweep the same blocks: equal bit for bit.
+packed heads sweep the same blocks: equal bit for bit.  With integer scores P,
+its sums and the merge's weights are exact: the exact result in every type.
 Shapes: single rows, rows that fill a tile with packed heads and ones that end
 in the middle of a head, keys that leave the last range short, causal rows that
 see nothing of a range, every Q-scale granularity, both layouts.
@@ -21,14 +24,16 @@ import torch
 from test_gpu_flash_vrow import _flash, _tiles
 
 pytestmark = pytest.mark.gpu
-E = {"fp16": 2.0 ** -11, "bf16": 2.0 ** -9}
+E = {"fp16": 2.0 ** -11, "bf16": 2.0 ** -8}
 DT = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
-EO = {"bf16": 2.0 ** -9, "fp16": 2.0 ** -11, "fp32": 2.0 ** -24}
+EO = {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11, "fp32": 2.0 ** -24}
 
 # (B, Hq, Hkv, Nq, Nkv, causal)
 SHAPES = [(1, 1, 1, 1, 65, False), (1, 4, 1, 1, 4097, False), (2, 6, 2, 37, 3000, False),
           (3, 8, 2, 32, 1000, False), (1, 12, 3, 127, 2111, False), (1, 2, 2, 130, 5000, False),
-          (1, 2, 1, 1500, 1500, True), (1, 3, 3, 777, 777, True)]
+          (1, 2, 1, 1500, 1500, True), (1, 3, 3, 777, 777, True), (1, 1, 1, 3, 900, False),
+          (16, 32, 4, 3, 777, False), (4, 24, 4, 37, 2000, False), (1, 3, 3, 1100, 1100, True)]
+ONE_SWEEP = [SHAPES[0], SHAPES[7]]  # no gain from ranges (of SHAPES[7] at D = 64); the others are split
 PACKED = [(64, 32, 8, 1, 200, False), (96, 18, 3, 5, 131, False), (64, 16, 2, 3, 700, False)]  # FP8 too
 
 
@@ -47,8 +52,9 @@ def _close(got, want, v, ep, eo):
     assert torch.isfinite(got).all()
     bound = 2 * ep * v.double().abs().max() + (2 * eo + 10 * 2.0 ** -11) * want.abs()
     worst = ((got - want).abs() / bound).max().item()
-    print(f"  worst error/bound {worst:.3f}")
-    assert worst <= 1.0
+    rel, limit = ((got - want).norm() / want.norm()).item(), 2 * ep / 3 ** 0.5 + 2 * eo + 10 * 2.0 ** -11
+    print(f"  worst error/bound {worst:.3f}, relative 2-norm {rel:.2e} of {limit:.2e}")
+    assert worst <= 1.0 and rel <= limit
 
 
 @pytest.mark.parametrize("D", [64, 128])
@@ -111,6 +117,43 @@ def test_flash_split_matches_one_sweep(shape, dtype, D, gpu_device):
     F = _flash()
     q, k, v = _inputs(shape, D, dtype, gpu_device)
     _close(F.run(q, k, v, causal=shape[5]), _tiles(F._H, q, k, v, shape[5]), v, E[dtype], EO[dtype])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("shape", SHAPES + PACKED, ids=lambda s: "-".join(str(int(x)) for x in s))
+def test_split_exact(shape, D, hip_impl, gpu_device):
+    """Scores in -2 .. 2: every P is one of five consecutive powers of two, 32
+    of which fp16 adds exactly, whatever maximum a range has.  A channel of 127
+    that the other operand does not have makes the INT8 scales 1."""
+    B, Hq, Hkv, Nq, Nkv, causal = shape
+    g = torch.Generator().manual_seed(Nkv + D)
+    q8, k8 = torch.zeros(B, Hq, Nq, D), torch.zeros(B, Hkv, Nkv, D)
+    q8[..., :2] = torch.randint(-1, 2, (B, Hq, Nq, 2), generator=g).float()
+    k8[..., :2] = torch.randint(-1, 2, (B, Hkv, Nkv, 2), generator=g).float()
+    v = torch.randint(-1, 2, (B, Hkv, Nkv, D), generator=g) * 2.0 ** torch.randint(0, 4, (B, Hkv, Nkv, D), generator=g)
+    v[:, :, 0] = 8.0  # FP8: every channel's scale is 8 / 448, its codes exact
+    s = (q8[..., :2].double().reshape(B, Hkv, -1, 2) @ k8[..., :2].double().transpose(2, 3)).reshape(B, Hq, Nq, Nkv)
+    if causal:
+        s.masked_fill_(torch.arange(Nkv)[None] > torch.arange(Nq)[:, None], float("-inf"))
+    p = torch.exp2(s).reshape(B, Hkv, -1, Nkv)
+    want = ((p @ v.double()) / p.sum(dim=3, keepdim=True)).reshape(B, Hq, Nq, D)
+    sm_scale = 1.0 / 1.44269504
+
+    def check(o, dtype):
+        torch.cuda.synchronize()
+        err = (o.double().cpu() - want).abs()
+        print(f"  max error {err.max():.2e}")
+        assert (err <= 1e-5 * (1.0 + want.abs()) + EO[dtype] * want.abs()).all()
+
+    F = _flash()
+    for dtype in ("fp16", "bf16"):
+        print(f"[split exact] {shape} D{D} flash {dtype}", flush=True)
+        check(F.run(*(t.to(DT[dtype]).to(gpu_device) for t in (q8, k8, v)), causal=causal, sm_scale=sm_scale), dtype)
+    q8[..., 2], k8[..., 3] = 127.0, 127.0
+    for pv, dtype in [("fp16", "fp32"), ("bf16", "fp32"), ("fp8", "fp32"), ("fp16", "fp16"), ("bf16", "bf16")]:
+        print(f"[split exact] {shape} D{D} {pv} {dtype}", flush=True)
+        check(hip_impl.run(*(t.to(DT[dtype]).to(gpu_device) for t in (q8, k8, v)), causal=causal, sm_scale=sm_scale,
+                           pv_dtype=pv, smooth_k=False), dtype)
 
 
 @pytest.mark.parametrize("D", [64, 128])

@@ -1,4 +1,4 @@
-"""GPU parity of the unquantized attention (flash_attn pack, C-ABI sage_flash_fwd).
+"""GPU parity of the unquantized attention (flash_attn pack, C-ABI sage_flash_run).
 
 1. Exactness: small-integer q and k (exact in fp16 / bf16; Q K^T exact in the
    fp32 MFMA accumulators), a score multiplier of exactly 1 (sm_scale =
@@ -88,8 +88,9 @@ SMALL = [
     (1, 3, 3, 1000, 1000, 128, "fp16", False),
     (1, 2, 1, 130, 700, 128, "bf16", False),
     (1, 2, 2, 1, 500, 64, "fp16", False),
-    # D = 64: 10 and 18 mask-free iterations (one 10-block trip; one trip and
-    # 8 single iterations)
+    # D = 64: 10 mask-free iterations (two trips of 4 and two single ones); split
+    # into 8 ranges of 3 blocks, the last short (every kernel and leftover:
+    # test_gpu_launches.py)
     (1, 2, 2, 896, 896, 64, "fp16", False),
     (1, 2, 1, 1408, 1408, 64, "bf16", False),
 ]
@@ -118,7 +119,9 @@ def test_flash_rising_scores(dtype, D, causal, flash, gpu_device):
     """Scores rising by about 2.5 log2 units per 64-key block (the queries
     share a direction the keys drift along): the running max moves again and
     again, so the mask-free loop redoes blocks whose P exceed its shortcut's
-    bound and rescales O lazily throughout; the reference pack's gate holds."""
+    bound and rescales O lazily throughout; the reference pack's gate holds.
+    (These shapes are split over the keys, so it is the merge that sees maxima
+    far apart; one sweep with rising scores is in test_gpu_launches.py.)"""
     print(f"[flash-rising] {dtype} D={D} causal={causal}", flush=True)
     from test_gpu_attn import rising_inputs
     q, k, v = (t.to(DT[dtype]) for t in rising_inputs(1, 2, 1000, D, 2.5, seed=D))

@@ -166,3 +166,30 @@ def test_stages_of_typical_calls(routes, hip_impl):
     ]:
         rc, got = run_call(routes, hip_impl, *shape, **kw)
         assert rc == 0 and (got[0]["quant_q"], got[0]["v"]) == (quant_q, v), (shape, kw, got)
+
+
+def test_gpu_launch_shapes_take_the_launch_they_name(routes, hip_impl):
+    from test_gpu_launches import LAUNCHES
+
+    for launch, shape, causal, dtype, pv in LAUNCHES:
+        flash = launch[0] == "flash"
+        kw = dict(flash=True) if flash else dict(pv=pv, fuse_q=int(launch[0] == "i8q"))
+        rc, got = run_call(routes, hip_impl, *shape, dtype=dtype, causal=causal, **kw)
+        assert rc == 0 and (got[-1]["launch"], got[-1]["nw"], got[-1]["wpe"]) == launch, (launch, shape, dtype, pv, got)
+        assert got[-1]["vrow"] == int(flash or dtype == pv), got
+
+
+def test_gpu_split_shapes_split(routes, hip_impl):
+    """The shapes that test_gpu_attn_split.py compares with one sweep are split, in both packs."""
+    from test_gpu_attn_split import ONE_SWEEP, SHAPES
+
+    packed = set()
+    for shape in SHAPES:
+        for D in (64, 128):
+            for kw in [dict(flash=True, dtype="fp16"), dict(flash=True), dict(dtype="bf16"), dict(dtype="fp32", pv="bf16"),
+                       dict(dtype="fp16", fuse_q=1)]:
+                rc, got = run_call(routes, hip_impl, *shape[:5], D, causal=shape[5], **kw)
+                assert rc == 0 and (got[-1]["nsplit"] > 1 or shape in ONE_SWEEP), (shape, D, kw, got)
+                if got[-1]["grp"] > 1:
+                    packed.add(shape)
+    assert len(packed) >= 3, packed
