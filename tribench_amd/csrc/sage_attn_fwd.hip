@@ -21,22 +21,25 @@ struct AttnPlan {
   bool part() const { return grp > 1 || nsplit > 1; }
 };
 
-// Chosen by the time each launch is expected to take (us): work-groups fill
-// 256 slots (8 waves) or 512 (4 waves, two to a CU) in rounds, a round costs
-// its start (Q, first tiles, epilogue) plus a time per 64-key block; the
-// partial kernels add the merge and its traffic.  The constants are fitted to
-// 285 shapes (both packs, 1 to 25000 rows and keys, up to 14 launches each):
-// the pick is 1.1 % slower than the best launch of each shape on average and
-// 19 % at worst, where 8 waves without a split would be 35 % on average.
-// What they stand for: 8 waves share every tile, which is worth 18 % per
-// block on a full chip at INT8 D = 128 (B4 H32 N4096: 931 us against 958);
-// 4 waves overlap one work-group's start with another's blocks and cut
-// the rows finer (B2 H32 N2048 causal: 136 us against 149; 226 keys: 291
-// against 332); splits and packed heads fill the chip when rows are few (one
+// Chosen by a model of each launch's cost: work-groups fill 256 slots (8 waves)
+// or 512 (4 waves, two to a CU) in rounds, a round costs its start (Q, first
+// tiles, epilogue) plus a cost per 64-key block; the partial kernels add the
+// merge and its traffic.  The unit is arbitrary: an attention takes 1.7 to 2.8
+// us for each, by type and shape, so the sums rank the launches of one call and
+// predict no times.  The constants were fitted to timed calls of both packs.
+// Over 110 other random calls, 811 launches timed (1 to 25000 rows and keys),
+// the pick is 1.4 % slower than the call's best launch on average and within
+// 5 % for 102 of them, 26 % at worst (unquantized causal, B2 H8 N2517 D64: 8
+// waves 43 us, 4 waves 34); 8 waves without a split are 50 % slower on average.
+// What the constants stand for: 8 waves share every tile, which is worth 3 % of
+// an attention on a full chip at INT8 D = 128 (B4 H32 N4096: 931 us a call
+// against 958); 4 waves overlap one work-group's start with another's blocks
+// and cut the rows finer (B2 H32 N2048 causal: 136 us against 149; 226 keys:
+// 291 against 332); splits and packed heads fill the chip when rows are few (one
 // row, 4 heads to a KV head, 8192 keys: 52 us against 146).
 static AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_t Nkv, int64_t D, bool causal,
                           bool i8, int pv_mode, int dtype, bool may_split) {
-  const double start8 = 5.2, start4 = 3.7, split_us = 4.2, merge_bytes_per_us = 7.4e6;
+  const double start8 = 5.2, start4 = 3.7, split_cost = 4.2, merge_bytes_per_unit = 7.4e6;
   double blk8 = i8 ? 0.50 : 0.48, blk4 = i8 ? 0.505 : 0.525;  // D = 64
   if (D == 128) {
     blk8 = !i8 ? 0.98 : pv_mode == SAGE_PV_F16 ? 0.64 : pv_mode == SAGE_PV_BF16 ? 0.90 : 0.565;
@@ -57,7 +60,7 @@ static AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Nq, int64_
     const int64_t wgs = (grp * Nq + 127) / 128 * (Hq / grp) * B * nsplit;
     // (a work-group that has its CU to itself takes 0.8 of a block's time)
     double c = sweep(wgs, 512, start4, wgs <= 256 ? 0.8 * blk4 : blk4, nsplit);
-    if (part) c += split_us + (double)(B * Hq * Nq * nsplit * D * 8) / merge_bytes_per_us;
+    if (part) c += split_cost + (double)(B * Hq * Nq * nsplit * D * 8) / merge_bytes_per_unit;
     if (c < t) {
       t = c;
       best.nw = 4;
@@ -407,10 +410,14 @@ static RunPlan run_plan(const sage_call* c) {
   RunPlan r;
   r.attn = attn_plan(c->B, c->Hq, c->Hkv, c->Nq, c->Nkv, c->D, c->causal != 0, true, (int)c->pv_mode, (int)c->dtype, true);
   // The prologue saves a pass over Q (written and read again) and lengthens
-  // each work-group's start: with more 128-row blocks than CUs it is 1 to 18 %
-  // faster per call (226 keys, B2 H48 N17776 D64: 267 us against 292), with
-  // fewer the start is what counts and the pre-pass is 1 to 9 % faster (B1 H18
-  // N159 D128: 24.6 us against 26.8).
+  // each work-group's start.  By 128-row blocks of Q, whole calls: many times
+  // the CUs, it is 3 to 15 % faster (226 keys, B2 H48 N17776 D64: 215 us
+  // against 249; B2 H32 N2048 D128: 140.5 against 145.5); fewer than the CUs,
+  // the start is what counts and the pre-pass is up to 11 % faster (B1 H18 N159
+  // D128: 18.6 us against 20.6).  Between, 257 to 512 blocks in one round of
+  // work-groups, they are within 3 % either way (B1 H24 N1333 D128 bf16 51.9
+  // prologue, 51.1 pre-pass; B1 H24 N2000 62.6 and 64.4; B1 H40 N900 D64 33.5
+  // and 33.1), so the line at the number of CUs costs nothing there.
   // (the prologue takes only what sage_attn_fwd_q does: q_fusable; it writes a
   // caller's Q8 with q's strides, which is the layout of fuse_q 1 alone)
   r.fuse_q = c->fuse_q < 0 ? (c->Nq + 127) / 128 * c->Hq * c->B > 256 && q_fusable(*c) && !c->q8 : c->fuse_q != 0;

@@ -15,16 +15,18 @@
 // triton_impl.py:137,145,147) are handled here.
 //
 // Organisation (CDNA4):
-//  * A work-group is 8 waves (2 per SIMD) of 32 query rows (one 32-row MFMA
-//    tile each) of one (batch, head): Q8 rows, S, P and the O^T accumulators
-//    (fp32, 32 x D) all live in arch VGPRs.
+//  * A work-group is 8 waves (2 per SIMD) or 4 (two work-groups to a CU, or
+//    three at D = 64: WPE waves per SIMD) of 32 query rows (one 32-row MFMA tile
+//    each) of one (batch, head), or of the query heads of one KV head (kPart):
+//    Q8 rows, S, P and the O^T accumulators (fp32, 32 x D) all live in arch VGPRs.
 //  * K8 rows and V^T rows reach LDS in tiles of 64 keys by direct global ->
-//    LDS loads (global_load_lds_dwordx4), two iterations ahead of their use, in
-//    a ring of K tiles and one of V tiles: no staging registers, no VALU work.
-//    V arrives already converted and transposed (sage_vtiles), so a tile is a
-//    plain copy; the unquantized kernel also takes V as it is (kVRow) and
-//    transposes in the operand read.  The 16-byte chunks of each LDS row are XOR-swizzled so that the
-//    operand reads of 16 consecutive lanes (rows) hit distinct banks.
+//    LDS loads (global_load_lds_dwordx4), two iterations ahead of their use (V
+//    tiles of the unquantized D = 128 kernel one), in a ring of K tiles and one
+//    of V tiles (TileRing): no staging registers, no VALU work.  V arrives already converted and
+//    transposed (sage_vtiles), so a tile is a plain copy, or, of the P.V type,
+//    as it is (kVRow), transposed in the operand read.  The 16-byte chunks of
+//    each LDS row are XOR-swizzled so that the operand reads of 16 consecutive
+//    lanes (rows) hit distinct banks.
 //  * Each wave waits (vmcnt) for exactly its own loads of the tile the next
 //    iteration reads, then meets the others at a barrier without a memory
 //    fence (__syncthreads' fence would drain the whole prefetch).
@@ -303,10 +305,9 @@ struct TileRing {
   static constexpr int kVA = NV > 2 ? 1 : 0;
 };
 
-// One work-group: 8 waves (2 per SIMD) of 32 query rows (one 32-row MFMA tile
-// each) of one (batch, head); Q rows, S, P and the O^T accumulators live in
-// arch VGPRs.  Tiles of 64 keys (K rows and V^T rows) reach LDS by direct
-// global -> LDS loads, two iterations ahead of their use (TileRing).
+// One work-group: NW waves (WPE per SIMD of a full CU) of 32 query rows (one
+// 32-row MFMA tile each).  kPart: one range of the keys for the rows of a.grp
+// query heads, its unnormalised O, max and sum to the workspace (attn_merge).
 template <int QKM, int D, int PVM, typename TO, int NW, int WPE, bool kVRow, bool kPart>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void attn_fwd_kernel(AttnArgs a) {
   constexpr int BM = 32 * NW;  // query rows per work-group
@@ -942,7 +943,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WP
   // all three; measured -1.9 % per launch at config 2, -1.2 % at config 4,
   // -3 to -4.5 % for fp16/bf16 QK at D = 64; with FP8 P it was slower, and
   // fp16/bf16 QK at D = 128 has no registers left for it).  Two iterations
-  // per trip swap the buffers' roles (ten at D = 64, where the ring slots are
+  // per trip swap the buffers' roles (four at D = 64, where the ring slots are
   // constants too).  sl as for fast_iter.
   constexpr bool kTwoS = WPE == 2 && ((kI8 && PVM == SAGE_PV_F16) || (!kI8 && D == 64));
   static_assert(!(kTwoS && PVM == SAGE_PV_FP8), "fused_iter uses the fp16/bf16 P shortcut of softmax_fast_on");

@@ -166,7 +166,8 @@ _raw_stream = (getattr(torch._C, "_cuda_getCurrentRawStream", None)
                or (lambda index: torch.cuda.current_stream(index).cuda_stream))
 
 
-def whole_call(fn, fn_bytes, what, q, k, v, o, layout, dims, mul, causal, pv_mode=0, q_sub=0, smooth_k=0, fuse_q=0, outs=None):
+def whole_call(fn, fn_bytes, what, q, k, v, o, layout, dims, mul, causal, pv_mode=0, q_sub=0, smooth_k=0, fuse_q=0,
+               outs=None):
     """Run sage_run / sage_flash_run: pack the sage_call, allocate the
     workspace it asks for and launch on the current stream.  dims = (B, Hq,
     Hkv, Nq, Nkv, D); outs: q8, q_scale, k8, k_scale, km, v_scale tensors."""
@@ -372,10 +373,11 @@ def q_sub_of(q_gran):
 
 
 def fuse_q_default(head_dim):
-    """Where stage calls (and run's intermediates) have Q quantized when the caller
-    does not say: in the attention kernel's prologue at D = 128 (measured 1-2 % faster per forward at
-    configurations 2 and 3, even at 5), in the pre-pass at D = 64 (the
-    prologue costs more than it saves there: 2 % slower at configuration 4)."""
+    """Where stage calls (and run's intermediates) have Q quantized when the
+    caller does not say: in the attention kernel's prologue at D = 128 (measured
+    1-2 % faster per forward at configurations 2 and 3, even at 5), in the
+    pre-pass at D = 64 (the prologue costs more than it saves there: 2 % slower
+    at configuration 4, with 8-wave work-groups)."""
     return head_dim == 128
 
 
@@ -522,6 +524,6 @@ def run(q, k, v, causal=False, sm_scale=None, *, pv_dtype="fp16", q_gran="block"
         if fuse_q and pre["q8"].stride() != q.stride():
             raise ValueError("sage_attn hip: invalid argument: q8_out must be int8 with q's strides")
         outs = [pre.get(key) for key in ("q8", "q_scale", "k8", "k_scale", "km", "v_scale")]
-    whole_call(lib.sage_run, lib.sage_run_workspace_bytes, "sage_run", q, k, v, o, tensor_layout, dims, mul, causal, PV_MODES[pv_dtype], q_sub,
-               int(bool(smooth_k)), -1 if fuse_q is None else int(bool(fuse_q)), outs)
+    whole_call(lib.sage_run, lib.sage_run_workspace_bytes, "sage_run", q, k, v, o, tensor_layout, dims, mul, causal,
+               PV_MODES[pv_dtype], q_sub, int(bool(smooth_k)), -1 if fuse_q is None else int(bool(fuse_q)), outs)
     return (o, pre) if return_intermediates else o
