@@ -7,8 +7,12 @@
  * product library libsage_attn.so does not.  It is for the phase-split
  * measurement of tribench_amd/trace_phases.py.
  *
- * After sage_trace_attach(buf, words) every attention launch of the library
- * (sage_attn_fwd, sage_attn_fwd_q, sage_flash_fwd) writes 16 words per wave
+ * After sage_trace_attach(buf, words) the stage calls (sage_attn_fwd,
+ * sage_attn_fwd_q, sage_flash_fwd) launch the kernel with 8 waves to a
+ * work-group, and so do sage_run and sage_flash_run, whose own launch follows
+ * untraced where it is another (4 waves, or split over the keys).  Without a
+ * buffer attached every call makes the product's launches.  Each 8-wave launch
+ * writes 16 words per wave
  * into buf, at ((blockIdx.x * 8 + wave) * 16): s_memtime at the kernel's
  * entry, the end of its prologue, after iteration 0, after the mask-free
  * loops, after the generic iterations and after the epilogue [0..5]; the
@@ -17,7 +21,8 @@
  * s_memrealtime (100 MHz) at entry and exit [9, 10]; HW_ID | XCC_ID << 32
  * [11]; the work-group's remapped index [12]; s_memtime after the
  * prologue's Q quantization and after its tile wait [13, 14] (0 for the
- * kernels that take Q8 from the pre-pass or fp16/bf16 Q); [15] is 0.  A launch
+ * kernels that take Q8 from the pre-pass or fp16/bf16 Q); 1 if the launch was
+ * made for the trace alone, in a call that takes another [15].  A launch
  * whose grid needs more than `words` fails with "invalid argument".
  * buf = NULL detaches.  Returns 0 on success.
  */

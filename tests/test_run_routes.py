@@ -19,12 +19,10 @@ DT = {"fp32": 0, "fp16": 1, "bf16": 2}
 BUF, Q8 = 1 << 20, 1 << 21  # addresses nothing reads
 
 
-@pytest.fixture(scope="module")
-def routes(tmp_path_factory, hip_impl):
+def _build_routes(out, hip_impl, *flags):
     hip_impl._load()  # (first: as a dependency of the stand-ins it would bind to them)
     so = hip_impl.library_path()
-    out = tmp_path_factory.mktemp("routes") / "run_routes.so"
-    subprocess.run([hip_build.hipcc(), *hip_build.COMMON, "-O0", "-w", "-shared", "-x", "hip",
+    subprocess.run([hip_build.hipcc(), *hip_build.COMMON, *flags, "-O0", "-w", "-shared", "-x", "hip",
                     str(HERE / "native" / "run_routes.cpp"), "-x", "none", str(so), f"-Wl,-rpath,{so.parent}",
                     "-Wl,-Bsymbolic", "-o", str(out)], check=True, capture_output=True)
     lib = ctypes.CDLL(str(out))
@@ -34,6 +32,11 @@ def routes(tmp_path_factory, hip_impl):
         getattr(lib, name + "_workspace_bytes").restype = ctypes.c_size_t
         getattr(lib, name + "_workspace_bytes").argtypes = [ctypes.c_char_p]
     return lib
+
+
+@pytest.fixture(scope="module")
+def routes(tmp_path_factory, hip_impl):
+    return _build_routes(tmp_path_factory.mktemp("routes") / "run_routes.so", hip_impl)
 
 
 def dense(H, N, D):
@@ -193,3 +196,23 @@ def test_gpu_split_shapes_split(routes, hip_impl):
                 if got[-1]["grp"] > 1:
                     packed.add(shape)
     assert len(packed) >= 3, packed
+
+
+def test_trace_build_launches_once_unless_traced(routes, hip_impl, tmp_path):
+    """The trace build times as the product does; only with a trace attached,
+    and where the product's launch is not of 8 waves, one of 8 waves is added."""
+    traced = _build_routes(tmp_path / "trace_routes.so", hip_impl, "-DSAGE_TRACE=2")
+    traced.sage_trace_attach.argtypes = [ctypes.c_void_p, ctypes.c_int64]
+    eight = (1, 24, 8, 1333, 1333, 128)
+    for shape, kw in [(eight, {}), ((2, 24, 8, 961, 961, 64), {}), ((2, 8, 2, 32, 3000, 128), {}),
+                      ((1, 24, 8, 1333, 2500, 128), dict(flash=True)), ((8, 32, 8, 1, 8192, 128), dict(flash=True))]:
+        want = run_call(routes, hip_impl, *shape, **kw)[1]
+        assert run_call(traced, hip_impl, *shape, **kw)[1] == want
+        assert traced.sage_trace_attach(BUF, 1 << 30) == 0
+        got = run_call(traced, hip_impl, *shape, **kw)[1]
+        assert traced.sage_trace_attach(None, 0) == 0
+        if want[-1]["nw"] == 8:
+            assert got == want
+        else:
+            assert got[:-2] == want[:-1] and got[-1] == want[-1] and got[-2]["nw"] == 8, got
+    assert run_call(routes, hip_impl, *eight)[1][-1]["nw"] == 8

@@ -178,7 +178,7 @@ static int attn_setup(AttnArgs& a, const char* who, const int64_t* q_strides, in
 // waves per work-group of the entry points that have no workspace
 static int stage_nw(AttnArgs& a, int64_t D, int pv_mode, int dtype) {
 #if SAGE_TRACE
-  return 8;
+  if (g_trace) return 8;  // what is traced
 #endif
   const AttnPlan p = attn_plan(a.B, a.Hq, a.Hkv, a.Nq, a.Nkv, D, a.causal != 0, true, pv_mode, dtype, false);
   a.wpe = p.wpe;
@@ -349,8 +349,11 @@ extern "C" int sage_flash_run(const sage_call* c, void* stream) {
   if (need && (!c->workspace || (size_t)c->workspace_bytes < need || (uintptr_t)c->workspace % 256 != 0))
     return fail("%s: invalid argument: workspace (%zu bytes, 256-byte aligned)", who, need);
   hipStream_t st = static_cast<hipStream_t>(stream);
-#if SAGE_TRACE  // the trace is of the 8-wave kernel; the planned launch then writes the output
-  if (int rc = launch_attn_flash(a, (int)c->D, (int)c->dtype, 8, st, who)) return rc;
+#if SAGE_TRACE  // only 8-wave launches are traced: another plan's writes the output after one of those
+  if (g_trace && (p.part() || p.nw != 8)) {
+    a.trace_extra = 1;
+    if (int rc = launch_attn_flash(a, (int)c->D, (int)c->dtype, 8, st, who)) return rc;
+  }
 #endif
   if (p.part()) {
     part_setup(a, p, c->D, static_cast<char*>(c->workspace));
@@ -525,9 +528,12 @@ extern "C" int sage_run(const sage_call* c, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   AttnArgs a{};
   if (int rc = attn_args(a, who, *c, dq, q8, q8_strides, qs, k8, k8_strides, ks, vt, vs)) return rc;
-#if SAGE_TRACE  // the trace is of the 8-wave kernel; the planned launch then writes the output
-  if (int rc = dq ? launch_attn_i8(a, (int)c->D, pv, dt, 8, st, who) : launch_attn_i8q(a, (int)c->D, pv, dt, 8, st, who))
-    return rc;
+#if SAGE_TRACE  // as in sage_flash_run
+  if (g_trace && (r.attn.part() || r.attn.nw != 8)) {
+    a.trace_extra = 1;
+    if (int rc = dq ? launch_attn_i8(a, (int)c->D, pv, dt, 8, st, who) : launch_attn_i8q(a, (int)c->D, pv, dt, 8, st, who))
+      return rc;
+  }
 #endif
   if (r.attn.part()) {
     part_setup(a, r.attn, c->D, ws + r.off_part);

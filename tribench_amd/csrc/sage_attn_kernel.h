@@ -96,6 +96,7 @@ struct AttnArgs {
   float2* part_ml; // [nsplit][B*Hq*Nq] that max (log2 units) and the sum of p
 #if SAGE_TRACE
   unsigned long long* trace;  // kTraceWords per wave, indexed by (blockIdx.x, wave)
+  int trace_extra;            // a launch made for the trace alone
 #endif
 };
 
@@ -107,7 +108,7 @@ struct AttnArgs {
 // counts, all and mask-free [8]; s_memrealtime (100 MHz) at entry and exit
 // [9, 10]; HW_ID and XCC_ID [11]; the work-group's remapped index [12];
 // s_memtime after the prologue's Q quantization (its Q rows awaited) and
-// after its tile wait [13, 14].
+// after its tile wait [13, 14]; whether the launch was made for the trace alone [15].
 constexpr int kTraceWords = 16;
 
 // the stamps' LDS (a function-scope array: only the kernels that call this
@@ -1169,6 +1170,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WP
   tr_put(11, (unsigned long long)__builtin_amdgcn_s_getreg((31 << 11) | 4) |
                  ((unsigned long long)__builtin_amdgcn_s_getreg((31 << 11) | 20) << 32));
   tr_put(12, (unsigned long long)wg);
+  tr_put(15, (unsigned long long)a.trace_extra);
   if constexpr (kTrace) {
     SAGE_WAIT_LGKM0();
     if (a.trace && lane < kTraceWords)

@@ -18,6 +18,10 @@ markdown:
   the gap between consecutive work-groups on one CU, the spread of the
   XCDs' end times.
 
+Only work-groups of 8 waves are traced.  Where the product takes another
+launch (4 waves to a work-group, or the keys split), the traced one is made
+beside it and the output says so.
+
 The trace build keeps its stamps in LDS and its barrier counters in SGPRs;
 its launch time is printed next to the product library's for the same
 configuration (alternating launches), so the perturbation is visible.
@@ -119,12 +123,16 @@ def analyse(T: np.ndarray) -> str:
     grid = T.shape[0]
     clock = total / ((rt1 - rt0) / 100e6)  # Hz, per wave
     wg_cycles = total.mean(axis=1)
+    if T[:, :, 15].any():
+        out = ["(the product takes another launch at this shape: work-groups of 4 waves, or the keys split)", ""]
+    else:
+        out = []
     names = ["prologue", "iteration 0", "mask-free loops", "generic iterations", "epilogue"]
     per = ph.mean(axis=(0, 1))
-    out = [f"work-groups: {grid}; waves: {grid * NW}; mean cycles per work-group (per wave, s_memtime): "
-           f"{wg_cycles.mean():.0f}; shader clock {np.median(clock) / 1e9:.3f} GHz (median over waves, "
-           f"{np.percentile(clock, 5) / 1e9:.3f}-{np.percentile(clock, 95) / 1e9:.3f} for 90 %)", "",
-           "| phase | cycles per wave | share |", "|---|---|---|"]
+    out += [f"work-groups: {grid}; waves: {grid * NW}; mean cycles per work-group (per wave, s_memtime): "
+            f"{wg_cycles.mean():.0f}; shader clock {np.median(clock) / 1e9:.3f} GHz (median over waves, "
+            f"{np.percentile(clock, 5) / 1e9:.3f}-{np.percentile(clock, 95) / 1e9:.3f} for 90 %)", "",
+            "| phase | cycles per wave | share |", "|---|---|---|"]
     for nm, v in zip(names, per):
         out.append(f"| {nm} | {v:.0f} | {100 * v / per.sum():.1f} % |")
     out.append(f"| total | {per.sum():.0f} | 100 % |")
