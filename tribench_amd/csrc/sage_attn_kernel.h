@@ -111,13 +111,6 @@ struct AttnArgs {
 // after its tile wait [13, 14]; whether the launch was made for the trace alone [15].
 constexpr int kTraceWords = 16;
 
-// the stamps' LDS (a function-scope array: only the kernels that call this
-// allocate it)
-template <int NW>
-__device__ __forceinline__ unsigned long long* trace_lds() {
-  __shared__ unsigned long long s[NW * kTraceWords];
-  return s;
-}
 #endif
 
 // Operand type of the QK product: INT8 with per-block scales (SageAttention;
@@ -344,15 +337,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WP
   // ring for reads of the direct-to-LDS load issued last and drains the
   // prefetch before them (an s_waitcnt vmcnt(0) per iteration).
   constexpr int QAMAX = kFQ ? NW * (int)sizeof(float) : 0;  // the waves' max|x| of Q
-  __shared__ __attribute__((aligned(1024))) char smem[RING + SINK + QAMAX];
 #if SAGE_TRACE
+  constexpr int STAMPS = NW * kTraceWords * 8;
+  constexpr bool kTrace = NW == 8 && !kPart && RING + SINK + QAMAX + STAMPS <= 160 * 1024;
+  __shared__ __attribute__((aligned(1024))) char smem[RING + SINK + QAMAX + (kTrace ? STAMPS : 0)];
   // stamps go to LDS as they are taken (kept in registers they would change
   // the kernel being measured; a global store would enter the vmcnt
   // accounting of the tile loads) and to the trace buffer at the end.  A
   // kernel whose tile ring leaves no room for them is not traced.
-  constexpr bool kTrace = NW == 8 && !kPart && RING + SINK + QAMAX + NW * kTraceWords * 8 <= 160 * 1024;
-  unsigned long long* tr_s = nullptr;
-  if constexpr (kTrace) tr_s = trace_lds<NW>();
+  unsigned long long* tr_s = reinterpret_cast<unsigned long long*>(smem + RING + SINK + QAMAX);
   // every lane stores the same wave-uniform value (no branch around the store)
   auto tr_put = [&](int i, unsigned long long v) __attribute__((always_inline)) {
     if constexpr (kTrace) tr_s[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kTraceWords + i] = v;
@@ -360,6 +353,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WP
   tr_put(0, __builtin_amdgcn_s_memtime());
   tr_put(9, __builtin_amdgcn_s_memrealtime());
   uint32_t tr_wait = 0, tr_wait_fast = 0, tr_n = 0;  // barrier cycles; counts (mask-free << 16)
+#else
+  __shared__ __attribute__((aligned(1024))) char smem[RING + SINK + QAMAX];
 #endif
 
   static_assert(!kPart || !kFQ, "partial kernels take Q8 from the pre-pass");
