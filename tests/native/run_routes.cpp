@@ -57,3 +57,7 @@ extern "C" const char* take_routes() {
   routes.clear();
   return out.c_str();
 }
+
+extern "C" int k_waves_pay(int64_t nblk, int64_t D, int vt_in_b, int pv_mode) {
+  return sage::k_waves_pay(nblk, D, vt_in_b, pv_mode);
+}

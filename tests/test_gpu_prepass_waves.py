@@ -1,4 +1,5 @@
-"""K quantized one block to a wave (1024 blocks or more, 2048 without V tiles) against one to a work-group.
+"""K quantized one block to a wave (1024 blocks or more, 2048 without V tiles; not
+beside FP8 V tiles at head dim 128) against one to a work-group.
 
 The same heads quantized sixteen at a time stay below that, so both
 roles run on the same data; every output is equal bit for bit.  Lengths leave

@@ -216,3 +216,17 @@ def test_trace_build_launches_once_unless_traced(routes, hip_impl, tmp_path):
         else:
             assert got[:-2] == want[:-1] and got[-1] == want[-1] and got[-2]["nw"] == 8, got
     assert run_call(routes, hip_impl, *eight)[1][-1]["nw"] == 8
+
+
+def test_k_blocks_by_wave_only_where_that_is_faster(routes):
+    """At head dim 128 the wave role takes its launch's other roles the registers:
+    FP8 V tiles there, and long calls, keep a work-group to a K block."""
+    def pay(nblk, D, vt_in_b, pv):
+        return bool(routes.k_waves_pay(ctypes.c_int64(nblk), ctypes.c_int64(D), vt_in_b, PV[pv]))
+
+    for nblk in (1024, 2048, 4448, 8192, 16384):
+        for pv in PV:
+            assert pay(nblk, 64, 1, pv) and pay(nblk, 64, 0, pv) == (nblk >= 2048)
+            assert pay(nblk, 128, 1, pv) == (pv != "fp8" and nblk < 8192)
+            assert pay(nblk, 128, 0, pv) == (2048 <= nblk < 8192)
+    assert not pay(1023, 64, 1, "fp16") and not pay(1023, 128, 1, "fp16")

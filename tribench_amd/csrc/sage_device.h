@@ -134,6 +134,23 @@ namespace sage {
 int fail(const char* fmt, ...);
 int check_launch(const char* what);
 
+// Whether launch B of the pre-pass quantizes 16-bit K one block to a wave
+// instead of one to a work-group; nblk: K blocks of the call, vt_in_b: V tiles
+// (of pv_mode's type) in the launch.  Pre-pass in us, work-group role -> wave role, bf16.
+// It takes 4 blocks to a CU to pay beside V tiles (512 blocks with fp16 tiles, D =
+// 128: 14.4 -> 15.2), 8 without, where it depends on the shape below (1024 blocks of
+// 4096 keys 16.6 -> 15.3, 1136 of short ones at D = 64 14.7 -> 15.5).  D = 64, from
+// there on 4 to 22 % less: 1024 blocks 15.0 -> 12.5, 16384 127 -> 114, with FP8 tiles
+// 215 -> 185.  D = 128, whose wave role takes 108 VGPRs and leaves the launch's other
+// roles half their waves: 1024 blocks 20.2 -> 17.9, 2048 without tiles 24.0 -> 20.3,
+// 4448 71.0 -> 68.0, but 8192 118 -> 118 (Q blocks beside 157 -> 160), 16384 229 ->
+// 231 (Q 300 -> 311); and FP8 tiles, bound by the VALU, lose at every size: 1024
+// 25.4 -> 26.7, 8192 164 -> 177, 16384 285 -> 317.
+inline bool k_waves_pay(int64_t nblk, int64_t D, bool vt_in_b, int pv_mode) {
+  if (D == 128 && (nblk >= 8192 || (vt_in_b && pv_mode == SAGE_PV_FP8))) return false;
+  return nblk >= (vt_in_b ? 1024 : 2048);
+}
+
 // sage_prepass (vt NULL) or sage_prepass_vt, reporting errors as `who`
 int prepass_any(const char* who, const void* q, const void* k, const void* v, int in_dtype, int64_t B, int64_t Hq,
                 int64_t Hkv, int64_t Nq, int64_t Nkv, int64_t D, const int64_t* q_strides, const int64_t* k_strides,

@@ -483,8 +483,8 @@ __device__ __forceinline__ void head_stats(const PrepassArgs& a, int64_t b, int6
 // A wave holds its whole block (64 rows x D, 64 or 128 bytes per lane and 32
 // rows), so the block's max is a wave reduction, without the barriers and
 // LDS atomics of quant_block, four blocks share the head's statistics, and
-// four times the bytes are in flight.  Same arithmetic, same bits.  K of B8
-// H32 N4096 D128 (0.40 GB read and written): 107 us -> 87, 4.6 TB/s.
+// four times the bytes are in flight.  Same arithmetic, same bits.  Pre-pass of
+// K alone 25.9 us -> 19.4 at B4 H16 N4096 D64, 39.8 -> 37.2 at D128 (k_waves_pay).
 // Lane l holds channels 16(l % CPR) .. +16 of rows l / CPR + (64 / CPR) j.
 template <typename T, int D>
 __device__ __forceinline__ void quant_k_waves(const PrepassArgs& a, int64_t r, float* km_s, float* vs_s) {
@@ -748,15 +748,8 @@ int sage::prepass_any(const char* who, const void* q, const void* k, const void*
   const bool vt_in_b = vt && (pv_mode == SAGE_PV_FP8 || (need_b && !do_q));
   a.n_vt_a = vt && !vt_in_b ? a.ntile * Hkv * B : 0;
   a.n_vt_b = vt_in_b ? a.ntile * Hkv * B : 0;
-  // A wave to a K block needs 4 blocks to a CU to pay beside V tiles, 8 without
-  // (that launch is bound by the role's latency, which is longer).  bf16,
-  // with fp16 V tiles, D = 128: 512 blocks 13.6 us against 14.8, 1024 21.7 ->
-  // 17.9, 4096 58 -> 53, 16384 252 -> 227; D = 64: 9.2 against 9.7, 13.5 -> 10.7,
-  // 32.5 -> 28.3, 120 -> 112.  Without them here: 1136 blocks 14.7 against 15.5 at
-  // D = 64, 1152 25.5 against 26.9 at 128; 2048 15.4 -> 11.5 and 25.8 -> 19.8.  (fp32
-  // would take 128 VGPRs for its loads alone and runs at 5.9 TB/s without.)
   a.k_waves = need_b && in_dtype != SAGE_DTYPE_F32 && blkq == 128 && blkk == 64 && !vrows &&
-              a.nkb * Hkv * B >= (vt_in_b ? 1024 : 2048);
+              k_waves_pay(a.nkb * Hkv * B, D, vt_in_b, pv_mode);
   a.n_kblk_b = need_b ? (a.k_waves ? (a.nkb + 3) / 4 : a.nkb) * Hkv * B : 0;
   if (a.n_stat + a.n_qblk_a + a.n_kblk_a + a.n_vt_a > 0x7FFFFFFF || a.n_kblk_b + a.n_qblk_b + a.n_vt_b > 0x7FFFFFFF)
     return fail("%s: invalid argument: grid too large", who);
