@@ -141,8 +141,8 @@ int check_launch(const char* what);
 // 128: 14.4 -> 15.2), 8 without, where it depends on the shape below (1024 blocks of
 // 4096 keys 16.6 -> 15.3, 1136 of short ones at D = 64 14.7 -> 15.5).  D = 64, from
 // there on 4 to 22 % less: 1024 blocks 15.0 -> 12.5, 16384 127 -> 114, with FP8 tiles
-// 215 -> 185.  D = 128, whose wave role takes 108 VGPRs and leaves the launch's other
-// roles half their waves: 1024 blocks 20.2 -> 17.9, 2048 without tiles 24.0 -> 20.3,
+// 215 -> 185.  D = 128, whose wave role takes 106 VGPRs and leaves the launch's other
+// roles 4 waves to a SIMD of 7: 1024 blocks 20.2 -> 17.9, 2048 without tiles 24.0 -> 20.3,
 // 4448 71.0 -> 68.0, but 8192 118 -> 118 (Q blocks beside 157 -> 160), 16384 229 ->
 // 231 (Q 300 -> 311); and FP8 tiles, bound by the VALU, lose at every size: 1024
 // 25.4 -> 26.7, 8192 164 -> 177, 16384 285 -> 317.

@@ -544,7 +544,7 @@ __device__ __forceinline__ void quant_k_waves(const PrepassArgs& a, int64_t r, f
 }
 
 // Roles: K blocks, then Q blocks, then (FP8 P.V) V tiles.
-// kWaves: the K roles are quant_k_waves (a kernel of its own: with its 108 VGPRs
+// kWaves: the K roles are quant_k_waves (a kernel of its own: with its 106 VGPRs
 // at D = 128 the other K role would have 4 work-groups to a CU instead of 7).
 template <typename T, int D, int NIQ, int NIK, bool kWaves>
 __global__ __launch_bounds__(kPrepassThreads) void prepass_b_kernel(PrepassArgs a) {
