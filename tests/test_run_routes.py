@@ -230,3 +230,22 @@ def test_k_blocks_by_wave_only_where_that_is_faster(routes):
             assert pay(nblk, 128, 1, pv) == (pv != "fp8" and nblk < 8192)
             assert pay(nblk, 128, 0, pv) == (2048 <= nblk < 8192)
     assert not pay(1023, 64, 1, "fp16") and not pay(1023, 128, 1, "fp16")
+
+
+def test_stage_calls_keep_8_waves_for_few_rows(routes, hip_impl):
+    """The stage calls cannot split keys; with a head's rows in one work-group
+    and a CU to each, head dim 128 keeps 8 waves (they share the tile loads)."""
+    i3 = ctypes.c_int64 * 3
+    p = ctypes.c_void_p(BUF)
+    routes.sage_attn_fwd.argtypes = hip_impl._load().sage_attn_fwd.argtypes
+    for (B, Hq, Hkv, Nq, Nkv, D), pv, nw in [
+        ((4, 6, 3, 58, 9570, 128), "fp16", 8), ((4, 6, 3, 128, 9570, 128), "bf16", 8), ((1, 2, 2, 1, 200, 128), "fp16", 8),
+        ((4, 6, 3, 58, 9570, 128), "fp8", 4), ((4, 6, 3, 58, 9570, 64), "fp16", 4), ((4, 6, 3, 129, 9570, 128), "fp16", 4),
+        ((16, 32, 8, 58, 4000, 128), "fp16", 4),
+    ]:
+        sq, sk = i3(*dense(Hq, Nq, D)), i3(*dense(Hkv, Nkv, D))
+        routes.take_routes()
+        assert routes.sage_attn_fwd(p, sq, p, p, sk, p, p, hip_impl.DTYPE_VTILES, None, p, p, DT["fp32"], sq, B, Hq, Hkv,
+                                    Nq, Nkv, D, 0, 128, 64, 128, PV[pv], None) == 0
+        got = json.loads(routes.take_routes())
+        assert got["nw"] == nw, (B, Hq, Nq, Nkv, D, pv, got)

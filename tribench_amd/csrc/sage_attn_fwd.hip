@@ -180,6 +180,13 @@ static int stage_nw(AttnArgs& a, int64_t D, int pv_mode, int dtype) {
 #if SAGE_TRACE
   if (g_trace) return 8;  // what is traced
 #endif
+  // A head's rows within one 4-wave work-group, each with a CU to itself: 4 waves
+  // have nothing to gain, and at D = 128 with fp16 or bf16 P the idle waves of 8
+  // are worth their share of the tile loads.  58 rows over 9570 keys, B4 H6: 108.6
+  // us against 114.0, fp32 outputs 107.9 against 159.9; over 1500, 25.2 against
+  // 26.2.  (At D = 64 4 waves are 1 to 4 % faster there, with FP8 P 0 to 7 %; the
+  // whole calls split such keys.)
+  if (D == 128 && pv_mode != SAGE_PV_FP8 && a.Nq <= 128 && (int64_t)a.B * a.Hq <= 256) return 8;
   const AttnPlan p = attn_plan(a.B, a.Hq, a.Hkv, a.Nq, a.Nkv, D, a.causal != 0, true, pv_mode, dtype, false);
   a.wpe = p.wpe;
   return p.nw;
